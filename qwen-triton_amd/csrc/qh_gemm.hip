@@ -1112,8 +1112,7 @@ int gemm_typed(int ta, int tb, int M, int N, int K, const void* A, int64_t lda, 
   constexpr int E = 16 / sizeof(T);
   const bool a_ok = aligned16(A) && lda % E == 0 && (ta ? M % E == 0 : K % E == 0);
   const bool b_ok = aligned16(B) && ldb % E == 0 && (tb ? N % E == 0 : K % E == 0);
-  // The tile kernels address the up to 16 rows of one load with a 32-bit byte offset per lane.
-  const bool tile_ok = a_ok && b_ok && lda < (1ll << 27) && ldb < (1ll << 27);
+  const bool tile_ok = a_ok && b_ok && lda < kTileMaxLd && ldb < kTileMaxLd;
   if constexpr (is_mfma_type) {
     // Decode path for small M (up to 128 rows: decode batches and short
     // prefills), both operands k-contiguous; wide outputs with M > 16 (the

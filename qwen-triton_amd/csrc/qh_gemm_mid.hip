@@ -95,9 +95,11 @@ extern "C" int qh_gemm_group(int64_t M, int64_t K, const void* A, int64_t lda, i
   QH_CHECK_ARG(dtype == QH_BF16 || dtype == QH_F16, "qh_gemm_group: bf16/f16 only");
   QH_CHECK_ARG(aligned16(A) && lda % 8 == 0 && lda >= K && K % 8 == 0,
                "qh_gemm_group: A must be 16-byte aligned with K, lda multiples of 8");
+  QH_CHECK_ARG(lda < kTileMaxLd, "qh_gemm_group: rows of A 2^27 or more elements apart");
   QH_CHECK_ARG(!gated || ldb[0] == ldb[1], "qh_gemm_group: gated products need one weight stride");
   for (int i = 0; i < count; ++i) {
     QH_CHECK_ARG(aligned16(B[i]) && ldb[i] % 8 == 0 && ldb[i] >= K, "qh_gemm_group: product %d: bad B", i);
+    QH_CHECK_ARG(ldb[i] < kTileMaxLd, "qh_gemm_group: product %d: rows of B 2^27 or more elements apart", i);
     QH_CHECK_ARG((gated && i == 1) || (C[i] != nullptr && ldc[i] >= N[i]), "qh_gemm_group: product %d: bad C", i);
     QH_CHECK_ARG(!gated || bias == nullptr || bias[i] == nullptr, "qh_gemm_group: gated products take no bias");
   }

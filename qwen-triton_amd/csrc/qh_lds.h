@@ -61,6 +61,11 @@ __device__ __forceinline__ uint32_t lds_addr(const void* p) {
   return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)p;
 }
 
+// Row strides (elements) below which the tile kernels reach the rows of one load, up to 15 of 16-bit and
+// 7 of fp32 elements past the load's scalar base, with a 32-bit byte offset per lane.
+constexpr int64_t kTileMaxLd = 1ll << 27;
+constexpr bool tile_reach_ok(int rows, int64_t ld, int elem) { return rows * ld * elem + 1024 <= 1ll << 32; }
+
 // s_waitcnt immediates (gfx9 encoding: vmcnt in [3:0] and [15:14], expcnt in
 // [6:4], lgkmcnt in [11:8]) that wait on one counter only.
 constexpr int waitcnt_vm(int n) { return (n & 0xF) | (((n >> 4) & 3) << 14) | (0x7 << 4) | (0xF << 8); }

@@ -38,6 +38,7 @@ struct NTile {
   static constexpr int W = 16 / CPR;       // rows per 256-byte bank window
   static constexpr int PW = ROWS / RPI / NW;  // DMA instructions per wave
   static_assert(PW >= 1 && (ROWS / RPI) % NW == 0, "tile height");
+  static_assert(tile_reach_ok(RPI - 1, kTileMaxLd, sizeof(T)), "lane offset");
 
   static __device__ __forceinline__ int sw(int r) { return (r / W) & (CPR - 1); }
   // Rows of instruction n are RPI n + lane / CPR with n = wid + NW i; RPI / W
@@ -138,6 +139,7 @@ struct TTile {
   static constexpr int NI = BK / RPI;
   static constexpr int PW = NI / NW;
   static_assert(CPR >= 4 && CPR <= 64 && PW >= 1 && NI % NW == 0 && NW * RPI % 4 == 0, "tile width");
+  static_assert(tile_reach_ok(RPI - 1, kTileMaxLd, sizeof(T)), "lane offset");
   // A fragment read touches 64 bytes of four k-rows. A k-row of 32 columns is a quarter of a
   // 256-byte bank window, so the four fill it; one of 64 columns is half, so rows kr and kr + 2
   // share banks; a wider one fills it, so all four do.

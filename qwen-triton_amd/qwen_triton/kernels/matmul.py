@@ -80,6 +80,10 @@ def linear_group_ok(x: torch.Tensor, weights: list[torch.Tensor]) -> bool:
                and w.stride(0) % 8 == 0 and w.data_ptr() % 16 == 0 for w in weights)
 
 
+# Rows further apart (elements) are past the 32-bit lane offsets of the grouped launch.
+_GROUP_MAX_STRIDE = 1 << 27
+
+
 def linear_group_rows_ok(x: torch.Tensor, weights: list[torch.Tensor],
                          biases: list[torch.Tensor | None] | None = None, gated: bool = False) -> bool:
     """True when ``linear_group`` can serve more than 128 rows of ``x`` in one launch
@@ -93,7 +97,8 @@ def linear_group_rows_ok(x: torch.Tensor, weights: list[torch.Tensor],
             and _GUARD.runtime_ok and _native.available()):
         return False
     if not all(w.dtype == x.dtype and w.device == x.device and w.dim() == 2 and w.shape[1] == k and w.stride(1) == 1
-               and w.stride(0) % 8 == 0 and w.data_ptr() % 16 == 0 for w in weights):
+               and w.stride(0) % 8 == 0 and w.stride(0) < _GROUP_MAX_STRIDE and w.data_ptr() % 16 == 0
+               for w in weights):
         return False
     if any(b is not None and (gated or b.shape != w.shape[:1] or b.stride(0) != 1 or b.dtype != x.dtype
                               or b.device != x.device) for w, b in zip(weights, biases or ())):
@@ -101,7 +106,7 @@ def linear_group_rows_ok(x: torch.Tensor, weights: list[torch.Tensor],
     if gated and weights[0].stride(0) != weights[1].stride(0):
         return False
     rows = _rows(x, k)  # (a view unless the rows have to be copied for any product)
-    if rows.stride(0) % 8 or rows.data_ptr() % 16:
+    if rows.stride(0) % 8 or rows.stride(0) >= _GROUP_MAX_STRIDE or rows.data_ptr() % 16:
         return False
     return bool(_native.call("qh_gemm_group_ok", rows.shape[0], len(weights),
                              ctypes.addressof(_group_plan(weights, biases)[2]), int(gated)))

@@ -111,3 +111,15 @@ def test_missing_library_is_loud_for_gpu_tensors(monkeypatch):
     monkeypatch.setattr(_native, "available", lambda: False)
     with pytest.raises(RuntimeError, match="could not be loaded"):
         guard.use_native(None, FakeCuda())
+
+
+@pytest.mark.parametrize("lda,ldb", [(1 << 27, 64), (64, 1 << 27)])
+def test_grouped_products_refuse_rows_past_their_lane_offsets(lda, ldb):
+    """The grouped launch reaches the rows of a load with 32-bit lane offsets: strides that would wrap
+    are an argument error before any launch."""
+    arr = lambda t, *v: (t * len(v))(*v)  # noqa: E731
+    b, c = arr(ctypes.c_void_p, 4096, 4096), arr(ctypes.c_void_p, 8192, 8192)
+    ldb_, n, ldc = arr(ctypes.c_int64, 64, ldb), arr(ctypes.c_int64, 3072, 3072), arr(ctypes.c_int64, 3072, 3072)
+    with pytest.raises(_native.NativeUnsupported, match="elements apart"):
+        _native.call("qh_gemm_group", 517, 64, 4096, lda, 2, ctypes.addressof(b), ctypes.addressof(ldb_),
+                     ctypes.addressof(n), ctypes.addressof(c), ctypes.addressof(ldc), None, 0, _native.BF16, 0)

@@ -367,3 +367,26 @@ def test_decode_prepare_of_a_middling_batch(B, Sk):
         # probabilities round to bf16 in another order of the keys; then one rounding each
         err = (outs[0][0].double() - outs[1][0].double()).abs()
         assert (err <= 3 * EPS[dt] * (kv[:, :, :, 1].double().abs().mean() + outs[1][0].double().abs())).all()
+
+
+# A prompt whose rows lie past the grouped launch's 32-bit lane offsets runs as separate products.
+def test_grouped_rows_far_apart():
+    from qwen_triton.kernels.matmul import linear_group_rows_ok
+    from qwen_triton.modules import QwenMLP
+
+    M, H, stride, dt = 161, 1024, 1 << 27, torch.bfloat16
+    if torch.cuda.mem_get_info()[0] < 60 << 30:
+        pytest.skip("needs 44 GB of device memory")
+    torch.manual_seed(0)
+    mlp = QwenMLP(H, 3072).to("cuda", dt).eval()
+    far = torch.empty(stride * (M - 1) + H, dtype=dt, device="cuda").as_strided((M, H), (stride, 1))
+    far.copy_(_rand(M, H, dtype=dt, seed=1))
+    near = far.contiguous()
+    with torch.no_grad():
+        weights = [mlp.gate_proj.weight, mlp.up_proj.weight]
+        assert linear_group_rows_ok(near, weights, gated=True) and not linear_group_rows_ok(far, weights, gated=True)
+        want, got = mlp(near).double(), mlp(far).double()
+    # the same roundings of fp32 sums in another order: three bf16 roundings that may fall the other way
+    assert (got - want).norm() <= 4 * EPS[dt] * want.norm()
+    del far
+    torch.cuda.empty_cache()
