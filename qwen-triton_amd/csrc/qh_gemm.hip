@@ -1131,8 +1131,10 @@ int gemm_typed(int ta, int tb, int M, int N, int K, const void* A, int64_t lda, 
       const int rc = qh_gemm_mid_dispatch(ta, tb, M, N, K, A, lda, B, ldb, C, ldc, bias, qh_dtype_of<T>(),
                                           qh_dtype_of<OT>(), st);
       if (rc != QH_GEMM_MID_NONE) return rc;
-      return qh_gemm_tile_dispatch(ta, tb, M, N, K, A, lda, B, ldb, C, ldc, bias, qh_dtype_of<T>(),
-                                   qh_dtype_of<OT>(), st);
+      // (split roles: k-contiguous rows further apart take the vector-ALU kernel)
+      if (lda < (ta ? kTileMaxLd : kTileMaxLdSplit) && ldb < (tb ? kTileMaxLd : kTileMaxLdSplit))
+        return qh_gemm_tile_dispatch(ta, tb, M, N, K, A, lda, B, ldb, C, ldc, bias, qh_dtype_of<T>(),
+                                     qh_dtype_of<OT>(), st);
     }
   } else if constexpr (std::is_same<OT, float>::value) {
     if (tile_ok) return qh_gemm_f32_dispatch(ta, tb, M, N, K, a, lda, b, ldb, c, ldc, bi, st);

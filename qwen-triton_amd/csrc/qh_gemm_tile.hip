@@ -1931,6 +1931,8 @@ extern "C" int qh_lmce_rows_fwd(const void* X, int64_t ldx, const void* W, int64
   QH_CHECK_ARG(aligned16(X) && aligned16(W) && aligned16(Z) && ldx % 8 == 0 && ldw % 8 == 0 && ldz % 8 == 0 &&
                    H % 8 == 0 && V % 8 == 0 && ldx >= H && ldw >= H && ldz >= V,
                "qh_lmce_rows_fwd: 16-byte aligned rows with H, V, ldx, ldw, ldz multiples of 8 required");
+  QH_CHECK_ARG(ldx < kTileMaxLdSplit && ldw < kTileMaxLdSplit,
+               "qh_lmce_rows_fwd: rows of X or W 2^25 or more elements apart");
   QH_CHECK_ARG(ws_bytes >= qh_lmce_rows_workspace(N, V), "qh_lmce_rows_fwd: workspace %lld < %lld",
                (long long)ws_bytes, (long long)qh_lmce_rows_workspace(N, V));
   QH_CHECK_ARG(lse != nullptr && loss_rows != nullptr, "qh_lmce_rows_fwd: lse and loss_rows are required");

@@ -64,6 +64,9 @@ __device__ __forceinline__ uint32_t lds_addr(const void* p) {
 // Row strides (elements) below which the tile kernels reach the rows of one load, up to 15 of 16-bit and
 // 7 of fp32 elements past the load's scalar base, with a 32-bit byte offset per lane.
 constexpr int64_t kTileMaxLd = 1ll << 27;
+// The same for a k-contiguous operand of a tile kernel with split load and store roles, whose loading
+// waves also reach the rows of another wave's load, 39 rows on.
+constexpr int64_t kTileMaxLdSplit = 1ll << 25;
 constexpr bool tile_reach_ok(int rows, int64_t ld, int elem) { return rows * ld * elem + 1024 <= 1ll << 32; }
 
 // s_waitcnt immediates (gfx9 encoding: vmcnt in [3:0] and [15:14], expcnt in

@@ -39,6 +39,7 @@ struct NTile {
   static constexpr int PW = ROWS / RPI / NW;  // DMA instructions per wave
   static_assert(PW >= 1 && (ROWS / RPI) % NW == 0, "tile height");
   static_assert(tile_reach_ok(RPI - 1, kTileMaxLd, sizeof(T)), "lane offset");
+  static constexpr int64_t kMaxLdSplit = kTileMaxLdSplit;
 
   static __device__ __forceinline__ int sw(int r) { return (r / W) & (CPR - 1); }
   // Rows of instruction n are RPI n + lane / CPR with n = wid + NW i; RPI / W
@@ -81,6 +82,7 @@ struct NTile {
   // scalar row address with the lane offset vo2 = vo + shift(ld) (at() linear in the
   // row with stride ld).
   static __device__ __forceinline__ uint32_t shift(int64_t ld) {
+    static_assert(tile_reach_ok(RPI - 1 + (NW / 2) * RPI, kMaxLdSplit, sizeof(T)), "lane offset");
     return (uint32_t)((int64_t)(NW / 2) * RPI * ld * (int64_t)sizeof(T));
   }
   template <class AT>
@@ -138,6 +140,7 @@ struct TTile {
   static constexpr int RPI = 64 / CPR;   // k-rows per 1 KiB instruction (64 lanes x 16 bytes)
   static constexpr int NI = BK / RPI;
   static constexpr int PW = NI / NW;
+  static constexpr int64_t kMaxLdSplit = kTileMaxLd;
   static_assert(CPR >= 4 && CPR <= 64 && PW >= 1 && NI % NW == 0 && NW * RPI % 4 == 0, "tile width");
   static_assert(tile_reach_ok(RPI - 1, kTileMaxLd, sizeof(T)), "lane offset");
   // A fragment read touches 64 bytes of four k-rows. A k-row of 32 columns is a quarter of a
@@ -185,6 +188,7 @@ struct TTile {
   // Split roles (as NTile::issue2): the instructions of wave wid + NW/2 read the
   // k-rows NW/2 RPI further on at the same swizzle.
   static __device__ __forceinline__ uint32_t shift(int64_t ld) {
+    static_assert(tile_reach_ok(RPI - 1 + (NW / 2) * RPI, kMaxLdSplit, sizeof(T)), "lane offset");
     return (uint32_t)((int64_t)(NW / 2) * RPI * ld * (int64_t)sizeof(T));
   }
   template <class AT>

@@ -123,3 +123,11 @@ def test_grouped_products_refuse_rows_past_their_lane_offsets(lda, ldb):
     with pytest.raises(_native.NativeUnsupported, match="elements apart"):
         _native.call("qh_gemm_group", 517, 64, 4096, lda, 2, ctypes.addressof(b), ctypes.addressof(ldb_),
                      ctypes.addressof(n), ctypes.addressof(c), ctypes.addressof(ldc), None, 0, _native.BF16, 0)
+
+
+@pytest.mark.parametrize("ldx,ldw", [(1 << 25, 64), (64, 1 << 25)])
+def test_fused_loss_refuses_rows_past_its_lane_offsets(ldx, ldw):
+    """The logits kernel's loading waves reach 39 rows past a load's base with 32-bit lane offsets."""
+    with pytest.raises(_native.NativeUnsupported, match="elements apart"):
+        _native.call("qh_lmce_rows_fwd", 4096, ldx, 4096, ldw, 4096, 512, 1024, 64, -100, 4096, 1024, 4096, 4096,
+                     4096, 1 << 30, _native.BF16, 0)

@@ -369,6 +369,28 @@ def test_decode_prepare_of_a_middling_batch(B, Sk):
         assert (err <= 3 * EPS[dt] * (kv[:, :, :, 1].double().abs().mean() + outs[1][0].double().abs())).all()
 
 
+# The same for the 256x256 tiles, whose loading waves reach rows 32 further on: the widest stride that they
+# take and the first that they do not.
+@pytest.mark.parametrize("stride", [(1 << 25) - 8, 1 << 25, 1 << 26])
+def test_gemm_large_output_of_rows_far_apart(stride):
+    from qwen_triton.kernels.matmul import gemm
+
+    M, N, K, dt = 256, 32776, 64, torch.bfloat16
+    if torch.cuda.mem_get_info()[0] < 50 << 30:
+        pytest.skip("needs 35 GB of device memory")
+    a = torch.empty(stride * (M - 1) + K, dtype=dt, device="cuda").as_strided((M, K), (stride, 1))
+    a.copy_(_rand(M, K, dtype=dt, seed=1))
+    b = _rand(N, K, dtype=dt, seed=2)
+    out = torch.empty(M, N, dtype=dt, device="cuda")
+    gemm(False, False, M, N, K, a, stride, b, K, out, N)
+    ad, bd = a.cpu().double(), b.cpu().double()
+    ref = ad @ bd.T
+    bound = (K + 1) * 2.0 ** -24 * (ad.abs() @ bd.T.abs()) + EPS[dt] * ref.abs()
+    assert ((out.cpu().double() - ref).abs() <= bound).all()
+    del a
+    torch.cuda.empty_cache()
+
+
 # A prompt whose rows lie past the grouped launch's 32-bit lane offsets runs as separate products.
 def test_grouped_rows_far_apart():
     from qwen_triton.kernels.matmul import linear_group_rows_ok
