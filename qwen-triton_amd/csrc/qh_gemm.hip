@@ -984,7 +984,7 @@ __global__ __launch_bounds__(256) void moe_stream_kernel(const T* __restrict__ A
     for (int i = 0; i < 2; ++i) {
       const int n = w + 4 * i;  // (rows past the last repeat it; their products are not stored)
       const int r = r0 + min(8 * n + rin, vr - 1);
-      ap[i] = A + (int64_t)(rows ? rows[r] : r) * lda + (n & 1 ? kc ^ 32 : kc);
+      ap[i] = A + (int64_t)(MODE == MOE_GATED ? rows[r] : r) * lda + (n & 1 ? kc ^ 32 : kc);
     }
     auto issue = [&](int kt) {
       const uint32_t base = lds0 + (uint32_t)((kt % NS) * STAGE * (int)sizeof(T));

@@ -412,3 +412,38 @@ def test_grouped_rows_far_apart():
     assert (got - want).norm() <= 4 * EPS[dt] * want.norm()
     del far
     torch.cuda.empty_cache()
+
+
+def _expert_gemm(mode, a, rows, table, ldb, n, wrow, seg, toff, E):
+    from qwen_triton import _native
+
+    R = int(seg[-1])
+    out = torch.full((R, n), 7.0, dtype=a.dtype, device="cuda")
+    _native.call("qh_moe_gemm", mode, a.data_ptr(), a.stride(0), None if rows is None else rows.data_ptr(),
+                 table.data_ptr(), ldb, out.data_ptr(), n, None if wrow is None else wrow.data_ptr(), seg.data_ptr(),
+                 toff.data_ptr(), R, E, n, a.shape[1], _native.dtype_code(a.dtype), _native.stream(a.device))
+    return out
+
+
+def _expert_segments(counts):
+    c = torch.tensor(counts)
+    zero = torch.zeros(1, dtype=torch.long)
+    return tuple(torch.cat((zero, x.cumsum(0))).to(torch.int32).cuda() for x in (c, (c + 127) // 128))
+
+
+# The scaled product's rows are contiguous whatever row list it is handed: few rows per expert (weights
+# streamed) and many (128-row tiles).
+@pytest.mark.parametrize("counts", [(5, 0, 40, 19), (200, 0, 150, 130)])
+def test_moe_scaled_product_reads_contiguous_rows(counts):
+    E, K, N, dt = len(counts), 128, 264, torch.bfloat16
+    seg, toff = _expert_segments(counts)
+    R = sum(counts)
+    a, w, down = _rand(R, K, dtype=dt, seed=1), _rand(R, dtype=dt, seed=2), _rand(E, N, K, dtype=dt, seed=3)
+    table = torch.tensor([down[e].data_ptr() for e in range(E)], dtype=torch.int64, device="cuda")
+    rows = (torch.arange(R, device="cuda") // 2).to(torch.int32)
+    want = _expert_gemm(1, a, None, table, K, N, w, seg, toff, E)
+    assert torch.equal(_expert_gemm(1, a, rows, table, K, N, w, seg, toff, E), want)
+    expert = torch.repeat_interleave(torch.arange(E), torch.tensor(counts))
+    ref = torch.einsum("rk,rnk->rn", a.cpu().double(), down.cpu().double()[expert]) * w.cpu().double()[:, None]
+    # the product and its scaled copy round once each
+    assert ((want.cpu().double() - ref).abs() <= 2.1 * EPS[dt] * ref.abs() + 1e-3).all()
