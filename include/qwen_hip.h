@@ -190,7 +190,7 @@ int qh_moe_dispatch(const int64_t* selected, const void* weights, int64_t n_toke
 /* Grouped expert GEMM over the dispatch segments (tile_off for tile_m = 128).
  * B_table is a DEVICE array of weight pointers ([out, in] row-major, row stride
  * ldb): mode 0 (gated): 2*E entries (gate_e, up_e), A = X gathered through
- * rows[], C[r] = silu(X[rows[r]] Wg^T) * (X[rows[r]] Wu^T), N = intermediate;
+ * rows[] (below 0: a row of zeros), C[r] = silu(X[rows[r]] Wg^T) * (X[rows[r]] Wu^T), N = intermediate;
  * mode 1 (scaled): E entries, A rows contiguous, C[r] = (A[r] Wd^T) * wrow[r].
  * Each product is rounded to the dtype before the SiLU-mul / scaling, as the
  * reference's per-expert TritonLinear, silu_mul and multiply do.

@@ -932,6 +932,7 @@ __global__ __launch_bounds__(256) void moe_gemm_kernel(const T* __restrict__ A, 
 // tile kernel / this one: 1 token 88 / 66, 16 233 / 166, 64 289 / 222, 512 (32 rows each) 324 / 273, 700
 // 343 / 294, 1024 358 / 453. 64 tokens read 1.2 GB: gate/up and down at 6.2 TB/s, 4.6 before.
 constexpr int64_t kMoeStreamRows = 48;
+__device__ const uint4 kMoeZeroChunk = {0, 0, 0, 0};
 
 template <typename T, int MODE>
 __global__ __launch_bounds__(256) void moe_stream_kernel(const T* __restrict__ A, int64_t lda,
@@ -979,19 +980,25 @@ __global__ __launch_bounds__(256) void moe_stream_kernel(const T* __restrict__ A
   const int nk = K / BK;
   for (int r0 = r_first; r0 < r_end; r0 += BMR) {
     const int vr = min(r_end - r0, BMR), nb = (vr + 15) >> 4;
-    const T* ap[2];
+    const T* ap[2];  // the next k-tile's chunk of the lane's row
+    int astep[2];
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
       const int n = w + 4 * i;  // (rows past the last repeat it; their products are not stored)
       const int r = r0 + min(8 * n + rin, vr - 1);
-      ap[i] = A + (int64_t)(MODE == MOE_GATED ? rows[r] : r) * lda + (n & 1 ? kc ^ 32 : kc);
+      const int src = MODE == MOE_GATED ? rows[r] : r;  // (below 0: a row of zeros)
+      ap[i] = src >= 0 ? A + (int64_t)src * lda + (n & 1 ? kc ^ 32 : kc) : reinterpret_cast<const T*>(&kMoeZeroChunk);
+      astep[i] = src >= 0 ? BK : 0;
     }
-    auto issue = [&](int kt) {
+    auto issue = [&](int kt) {  // (k-tiles in order)
       const uint32_t base = lds0 + (uint32_t)((kt % NS) * STAGE * (int)sizeof(T));
 #pragma unroll
       for (int i = 0; i < 4; ++i) lds_dma16_nt(bp[i] + kt * BK, base + (uint32_t)(4 * w + i) * 1024u);
 #pragma unroll
-      for (int i = 0; i < 2; ++i) lds_dma16(ap[i] + kt * BK, base + (uint32_t)(16 + w + 4 * i) * 1024u);
+      for (int i = 0; i < 2; ++i) {
+        lds_dma16(ap[i], base + (uint32_t)(16 + w + 4 * i) * 1024u);
+        ap[i] += astep[i];
+      }
     };
     f32x4 acc[4][2];
 #pragma unroll

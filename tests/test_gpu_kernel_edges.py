@@ -447,3 +447,20 @@ def test_moe_scaled_product_reads_contiguous_rows(counts):
     ref = torch.einsum("rk,rnk->rn", a.cpu().double(), down.cpu().double()[expert]) * w.cpu().double()[:, None]
     # the product and its scaled copy round once each
     assert ((want.cpu().double() - ref).abs() <= 2.1 * EPS[dt] * ref.abs() + 1e-3).all()
+
+
+# A row list entry below 0 is a row of zeros, in the first, a middle and the last place of a segment.
+@pytest.mark.parametrize("counts", [(5, 0, 40, 19), (200, 0, 150, 130)])
+def test_moe_gated_product_of_missing_rows(counts):
+    E, K, N, dt = len(counts), 128, 136, torch.bfloat16
+    seg, toff = _expert_segments(counts)
+    R, T = sum(counts), 30
+    x, gu = _rand(T, K, dtype=dt, seed=1), _rand(2 * E, N, K, dtype=dt, seed=3, scale=0.2)
+    table = torch.tensor([w.data_ptr() for w in gu], dtype=torch.int64, device="cuda")
+    rows = torch.arange(R, device="cuda") % T
+    want = _expert_gemm(0, x, rows.to(torch.int32), table, K, N, None, seg, toff, E)
+    gone = torch.tensor([0, 2, 4, 5, 17, R - 1], device="cuda")
+    rows[gone] = -1
+    got = _expert_gemm(0, x, rows.to(torch.int32), table, K, N, None, seg, toff, E)
+    want[gone] = 0
+    assert torch.equal(got, want)
