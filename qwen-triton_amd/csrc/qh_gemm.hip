@@ -797,27 +797,33 @@ struct RowTileLoader {
   static __device__ __forceinline__ int row_of(int i) { return (threadIdx.x + i * 256) >> 3; }
 };
 
-template <typename T, int MODE>
-__global__ __launch_bounds__(256) void moe_gemm_kernel(const T* __restrict__ A, int64_t lda,
-                                                       const int* __restrict__ rows, const T* const* __restrict__ Bt,
-                                                       int64_t ldb, T* __restrict__ C, int64_t ldc,
-                                                       const T* __restrict__ wrow, const int* __restrict__ seg,
-                                                       const int* __restrict__ toff, int E, int N, int K) {
-  constexpr int BM = 128, BN = 128, WM = 2, WN = 2;
-  constexpr int WTM = BM / WM, WTN = BN / WN, TM = WTM / 32, TN = WTN / 32;
-  typedef typename Mfma<T>::v8 v8;
-  __shared__ __attribute__((aligned(16))) T smem[2][(BM + BN) * LDS_LD];
-
-  const int tm = blockIdx.x;
-  if (tm >= toff[E]) return;
+// Expert and rows [r0, r1) of M-tile tm of 128 rows; false past the last tile.
+__device__ __forceinline__ bool moe_tile_rows(const int32_t* __restrict__ seg, const int32_t* __restrict__ toff, int E,
+                                              int tm, int& e, int& r0, int& r1) {
+  if (tm >= toff[E]) return false;
   int lo = 0, hi = E;  // largest e with toff[e] <= tm
   while (hi - lo > 1) {
     const int mid = (lo + hi) >> 1;
     if (toff[mid] <= tm) lo = mid;
     else hi = mid;
   }
-  const int e = lo;
-  const int r0 = seg[e] + (tm - toff[e]) * BM, r1 = seg[e + 1];
+  e = lo;
+  r0 = seg[e] + (tm - toff[e]) * 128;
+  r1 = min(seg[e + 1], r0 + 128);
+  return true;
+}
+
+constexpr int kMoeTileLds = 2 * (128 + 128) * LDS_LD;  // elements
+// One 128-row tile on 128 weight rows.
+template <typename T, int MODE>
+__device__ __forceinline__ void moe_row_tile(T* lds, const T* __restrict__ A, int64_t lda,
+                                             const int32_t* __restrict__ rows, const T* const* __restrict__ Bt,
+                                             int64_t ldb, T* __restrict__ C, int64_t ldc, const T* __restrict__ wrow,
+                                             int e, int r0, int r1, int N, int K) {
+  constexpr int BM = 128, BN = 128, WM = 2, WN = 2;
+  constexpr int WTM = BM / WM, WTN = BN / WN, TM = WTM / 32, TN = WTN / 32;
+  typedef typename Mfma<T>::v8 v8;
+  auto stage = [&](int buf) { return lds + buf * ((BM + BN) * LDS_LD); };
   // MOE_GATED covers 64 output columns (gate and up), MOE_SCALED 128.
   const int n0 = blockIdx.y * (MODE == MOE_GATED ? 64 : 128);
 
@@ -856,8 +862,8 @@ __global__ __launch_bounds__(256) void moe_gemm_kernel(const T* __restrict__ A, 
   const int nk = (K + BK - 1) / BK;
   la.load(0, K);
   lb.load(0, K);
-  la.store(smem[0]);
-  lb.store(smem[0] + BM * LDS_LD);
+  la.store(stage(0));
+  lb.store(stage(0) + BM * LDS_LD);
   __syncthreads();
   for (int kt = 0; kt < nk; ++kt) {
     const int buf = kt & 1;
@@ -866,8 +872,8 @@ __global__ __launch_bounds__(256) void moe_gemm_kernel(const T* __restrict__ A, 
       la.load((kt + 1) * BK, K);
       lb.load((kt + 1) * BK, K);
     }
-    const T* As = smem[buf];
-    const T* Bs = smem[buf] + BM * LDS_LD;
+    const T* As = stage(buf);
+    const T* Bs = stage(buf) + BM * LDS_LD;
 #pragma unroll
     for (int kk = 0; kk < BK / 16; ++kk) {
       v8 af[TM], bf[TN];
@@ -884,8 +890,8 @@ __global__ __launch_bounds__(256) void moe_gemm_kernel(const T* __restrict__ A, 
         for (int j = 0; j < TN; ++j) acc[i][j] = Mfma<T>::mma(af[i], bf[j], acc[i][j]);
     }
     if (more) {
-      la.store(smem[buf ^ 1]);
-      lb.store(smem[buf ^ 1] + BM * LDS_LD);
+      la.store(stage(buf ^ 1));
+      lb.store(stage(buf ^ 1) + BM * LDS_LD);
     }
     __syncthreads();
   }
@@ -918,44 +924,50 @@ __global__ __launch_bounds__(256) void moe_gemm_kernel(const T* __restrict__ A, 
   }
 }
 
+template <typename T, int MODE>
+__global__ __launch_bounds__(256) void moe_gemm_kernel(const T* __restrict__ A, int64_t lda,
+                                                       const int32_t* __restrict__ rows,
+                                                       const T* const* __restrict__ Bt, int64_t ldb,
+                                                       T* __restrict__ C, int64_t ldc, const T* __restrict__ wrow,
+                                                       const int32_t* __restrict__ seg,
+                                                       const int32_t* __restrict__ toff, int E, int N, int K) {
+  __shared__ __attribute__((aligned(16))) T smem[kMoeTileLds];
+  int e, r0, r1;
+  if (!moe_tile_rows(seg, toff, E, blockIdx.x, e, r0, r1)) return;
+  moe_row_tile<T, MODE>(smem, A, lda, rows, Bt, ldb, C, ldc, wrow, e, r0, r1, N, K);
+}
+
 // ---------------------------------------------------------------------------
 // The same for few rows per expert (a decode batch routed over many experts): bound by reading each
 // hit expert's weights once, so the work is a stream of weight rows against one small block of
 // activation rows. A workgroup takes 128 weight rows; each of its 4 wavefronts streams 32 of them,
 // non-temporally and NS - 1 k-tiles of 64 ahead, into its own part of an LDS ring (two workgroups per
-// CU keep 64 KB of weights in flight), beside the expert's first 64 rows, shared, of which only the
+// CU keep 64 KB of weights in flight), beside the tile's up to 64 rows, shared, of which only the
 // 16-row blocks in use are multiplied (16x16x32 MFMA). GATED wavefronts hold 16 gate and the same 16
-// up columns, so the SiLU-mul stays in the lane. A tile of more than 64 rows takes a second pass.
+// up columns, so the SiLU-mul stays in the lane.
 // ---------------------------------------------------------------------------
-// Rows per expert, on average, up to which it is taken (beyond, more and more tiles hold over 64 rows
-// and stream their weights twice). Expert path, us, 30B-A3B shapes (128 experts of 768, 8 per token),
-// tile kernel / this one: 1 token 88 / 66, 16 233 / 166, 64 289 / 222, 512 (32 rows each) 324 / 273, 700
-// 343 / 294, 1024 358 / 453. 64 tokens read 1.2 GB: gate/up and down at 6.2 TB/s, 4.6 before.
+// Rows of an expert that the stream takes. The tiles of a fuller one run as 128-row tiles, which read the
+// weights through L2, once for 128 rows: where a router sends its tokens to few experts, the average
+// says nothing of that. (768 tokens on 8 / 16 / 32 of
+// 128 experts, 8 each: streamed in passes of 64 rows 264 / 283 / 277 us, as 128-row tiles 175 / 185 / 201.)
+constexpr int kMoeStreamTile = 64, kMoeStreamStages = 3;
+// Rows per expert, on average, up to which the kernel with both is taken: beyond, hardly an expert is left
+// to stream. Expert path with its dispatch and combine, us, 30B-A3B shapes (128 experts of 768, 8 per
+// token), 128-row tiles behind a sort / this one behind moe_dispatch_small up to 256 tokens: 1 token 81 /
+// 46, 16 218 / 144, 64 264 / 199, 512 (32 rows each) 297 / 264, 700 319 / 284. 64 tokens read 1.2 GB:
+// gate/up and down at 6.2 TB/s, 4.6 before.
 constexpr int64_t kMoeStreamRows = 48;
+constexpr int kMoeStreamLds = kMoeStreamStages * (128 + kMoeStreamTile) * BK;  // elements
+static_assert(kMoeStreamLds >= kMoeTileLds, "either tile");
 __device__ const uint4 kMoeZeroChunk = {0, 0, 0, 0};
 
 template <typename T, int MODE>
-__global__ __launch_bounds__(256) void moe_stream_kernel(const T* __restrict__ A, int64_t lda,
-                                                         const int32_t* __restrict__ rows,
-                                                         const T* const* __restrict__ Bt, int64_t ldb,
-                                                         T* __restrict__ C, int64_t ldc, const T* __restrict__ wrow,
-                                                         const int32_t* __restrict__ seg,
-                                                         const int32_t* __restrict__ toff, int E, int N, int K) {
+__device__ __forceinline__ void moe_stream_tile(T* smem, const T* __restrict__ A, int64_t lda,
+                                                const int32_t* __restrict__ rows, const T* const* __restrict__ Bt,
+                                                int64_t ldb, T* __restrict__ C, int64_t ldc,
+                                                const T* __restrict__ wrow, int e, int r0, int r1, int N, int K) {
   typedef typename Mfma<T>::v8 v8;
-  constexpr int NS = 3, BMR = 64, STAGE = (128 + BMR) * BK;
-  extern __shared__ __attribute__((aligned(1024))) unsigned char qh_moe_smem[];
-  T* smem = reinterpret_cast<T*>(qh_moe_smem);
-  const int mt = blockIdx.x;
-  if (mt >= toff[E]) return;
-  int lo = 0, hi = E;  // expert of the tile: the last e with toff[e] <= mt
-  while (hi - lo > 1) {
-    const int mid = (lo + hi) >> 1;
-    if (toff[mid] <= mt) lo = mid;
-    else hi = mid;
-  }
-  const int e = lo;
-  const int r_first = seg[e] + (mt - toff[e]) * 128;
-  const int r_end = min(seg[e + 1], r_first + 128);
+  constexpr int NS = kMoeStreamStages, BMR = kMoeStreamTile, STAGE = (128 + BMR) * BK;
   const int lane = threadIdx.x & 63, q = lane >> 4, c16 = lane & 15;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const uint32_t lds0 = lds_addr(smem);
@@ -978,81 +990,93 @@ __global__ __launch_bounds__(256) void moe_stream_kernel(const T* __restrict__ A
     bp[i] = W + (int64_t)min(col, N - 1) * ldb + (i & 1 ? kc ^ 32 : kc);
   }
   const int nk = K / BK;
-  for (int r0 = r_first; r0 < r_end; r0 += BMR) {
-    const int vr = min(r_end - r0, BMR), nb = (vr + 15) >> 4;
-    const T* ap[2];  // the next k-tile's chunk of the lane's row
-    int astep[2];
+  const int vr = r1 - r0, nb = (vr + 15) >> 4;
+  const T* ap[2];  // the next k-tile's chunk of the lane's row
+  int astep[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int n = w + 4 * i;  // (rows past the last repeat it; their products are not stored)
+    const int r = r0 + min(8 * n + rin, vr - 1);
+    const int src = MODE == MOE_GATED ? rows[r] : r;  // (below 0: a row of zeros)
+    ap[i] = src >= 0 ? A + (int64_t)src * lda + (n & 1 ? kc ^ 32 : kc) : reinterpret_cast<const T*>(&kMoeZeroChunk);
+    astep[i] = src >= 0 ? BK : 0;
+  }
+  auto issue = [&](int kt) {  // (k-tiles in order)
+    const uint32_t base = lds0 + (uint32_t)((kt % NS) * STAGE * (int)sizeof(T));
+#pragma unroll
+    for (int i = 0; i < 4; ++i) lds_dma16_nt(bp[i] + kt * BK, base + (uint32_t)(4 * w + i) * 1024u);
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
-      const int n = w + 4 * i;  // (rows past the last repeat it; their products are not stored)
-      const int r = r0 + min(8 * n + rin, vr - 1);
-      const int src = MODE == MOE_GATED ? rows[r] : r;  // (below 0: a row of zeros)
-      ap[i] = src >= 0 ? A + (int64_t)src * lda + (n & 1 ? kc ^ 32 : kc) : reinterpret_cast<const T*>(&kMoeZeroChunk);
-      astep[i] = src >= 0 ? BK : 0;
+      lds_dma16(ap[i], base + (uint32_t)(16 + w + 4 * i) * 1024u);
+      ap[i] += astep[i];
     }
-    auto issue = [&](int kt) {  // (k-tiles in order)
-      const uint32_t base = lds0 + (uint32_t)((kt % NS) * STAGE * (int)sizeof(T));
+  };
+  f32x4 acc[4][2];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) lds_dma16_nt(bp[i] + kt * BK, base + (uint32_t)(4 * w + i) * 1024u);
+  for (int i = 0; i < 4; ++i)
 #pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        lds_dma16(ap[i], base + (uint32_t)(16 + w + 4 * i) * 1024u);
-        ap[i] += astep[i];
-      }
+    for (int j = 0; j < 2; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int t = 0; t < NS - 1; ++t)
+    if (t < nk) issue(t);
+  for (int kt = 0; kt < nk; ++kt) {
+    if (kt + 1 < nk) __builtin_amdgcn_s_waitcnt(waitcnt_vm(6));
+    else __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
+    __syncthreads();  // k-tile kt has landed for every wave, and every wave has read k-tile kt - 1
+    if (kt + NS - 1 < nk) issue(kt + NS - 1);
+    const T* S = smem + (kt % NS) * STAGE;
+    const T* Sa = S + 128 * BK;
+    auto frag = [&](const T* P, int row, int kk) {
+      return *reinterpret_cast<const v8*>(P + row * BK + 8 * ((4 * kk + q) ^ ((row >> 1) & 7)));
     };
-    f32x4 acc[4][2];
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int kk = 0; kk < 2; ++kk) {
+      const v8 b0 = frag(S, 32 * w + c16, kk), b1 = frag(S, 32 * w + 16 + c16, kk);
 #pragma unroll
-      for (int j = 0; j < 2; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int t = 0; t < NS - 1; ++t)
-      if (t < nk) issue(t);
-    for (int kt = 0; kt < nk; ++kt) {
-      if (kt + 1 < nk) __builtin_amdgcn_s_waitcnt(waitcnt_vm(6));
-      else __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
-      __syncthreads();  // k-tile kt has landed for every wave, and every wave has read k-tile kt - 1
-      if (kt + NS - 1 < nk) issue(kt + NS - 1);
-      const T* S = smem + (kt % NS) * STAGE;
-      const T* Sa = S + 128 * BK;
-      auto frag = [&](const T* P, int row, int kk) {
-        return *reinterpret_cast<const v8*>(P + row * BK + 8 * ((4 * kk + q) ^ ((row >> 1) & 7)));
-      };
-#pragma unroll
-      for (int kk = 0; kk < 2; ++kk) {
-        const v8 b0 = frag(S, 32 * w + c16, kk), b1 = frag(S, 32 * w + 16 + c16, kk);
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          if (i < nb) {
-            const v8 a = frag(Sa, 16 * i + c16, kk);
-            acc[i][0] = mma16<T>(a, b0, acc[i][0]);
-            acc[i][1] = mma16<T>(a, b1, acc[i][1]);
-          }
-      }
+      for (int i = 0; i < 4; ++i)
+        if (i < nb) {
+          const v8 a = frag(Sa, 16 * i + c16, kk);
+          acc[i][0] = mma16<T>(a, b0, acc[i][0]);
+          acc[i][1] = mma16<T>(a, b1, acc[i][1]);
+        }
     }
-    __syncthreads();  // the stages are free for the next pass
-    // accumulators: column c16, rows 4 q + r
+  }
+  // accumulators: column c16, rows 4 q + r
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < 4; ++i)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int row = 16 * i + 4 * q + r;
-        if (row >= vr) continue;
-        T* cr = C + (int64_t)(r0 + row) * ldc;
-        if constexpr (MODE == MOE_GATED) {
-          const int col = blockIdx.y * 64 + 16 * w + c16;
-          const float g = to_f32((T)acc[i][0][r]), u = to_f32((T)acc[i][1][r]);
-          if (col < N) cr[col] = from_f32<T>(g * sigmoidf_(g) * u);
-        } else {
-          const float ws = to_f32(wrow[r0 + row]);
+    for (int r = 0; r < 4; ++r) {
+      const int row = 16 * i + 4 * q + r;
+      if (row >= vr) continue;
+      T* cr = C + (int64_t)(r0 + row) * ldc;
+      if constexpr (MODE == MOE_GATED) {
+        const int col = blockIdx.y * 64 + 16 * w + c16;
+        const float g = to_f32((T)acc[i][0][r]), u = to_f32((T)acc[i][1][r]);
+        if (col < N) cr[col] = from_f32<T>(g * sigmoidf_(g) * u);
+      } else {
+        const float ws = to_f32(wrow[r0 + row]);
 #pragma unroll
-          for (int j = 0; j < 2; ++j) {
-            const int col = blockIdx.y * 128 + 32 * w + 16 * j + c16;
-            if (col < N) cr[col] = from_f32<T>(to_f32((T)acc[i][j][r]) * ws);
-          }
+        for (int j = 0; j < 2; ++j) {
+          const int col = blockIdx.y * 128 + 32 * w + 16 * j + c16;
+          if (col < N) cr[col] = from_f32<T>(to_f32((T)acc[i][j][r]) * ws);
         }
       }
-  }
+    }
+}
+
+template <typename T, int MODE>
+__global__ __launch_bounds__(256) void moe_stream_kernel(const T* __restrict__ A, int64_t lda,
+                                                         const int32_t* __restrict__ rows,
+                                                         const T* const* __restrict__ Bt, int64_t ldb,
+                                                         T* __restrict__ C, int64_t ldc, const T* __restrict__ wrow,
+                                                         const int32_t* __restrict__ seg,
+                                                         const int32_t* __restrict__ toff, int E, int N, int K) {
+  extern __shared__ __attribute__((aligned(1024))) unsigned char qh_moe_smem[];
+  T* smem = reinterpret_cast<T*>(qh_moe_smem);
+  int e, r0, r1;
+  if (!moe_tile_rows(seg, toff, E, blockIdx.x, e, r0, r1)) return;
+  if (seg[e + 1] - seg[e] <= kMoeStreamTile) moe_stream_tile<T, MODE>(smem, A, lda, rows, Bt, ldb, C, ldc, wrow, e, r0, r1, N, K);
+  else moe_row_tile<T, MODE>(smem, A, lda, rows, Bt, ldb, C, ldc, wrow, e, r0, r1, N, K);
 }
 
 // ---------------------------------------------------------------------------
@@ -1345,7 +1369,7 @@ extern "C" int qh_moe_gemm(int mode, const void* A, int64_t lda, const int32_t* 
   QH_CHECK_ARG(mt < (1ll << 31) && nt < 65536, "qh_moe_gemm: too many tiles");
   dim3 grid((unsigned)mt, (unsigned)nt);
   if (R <= kMoeStreamRows * E && K % BK == 0) {
-    constexpr int lds = 3 * (128 + 64) * BK * 2;
+    constexpr int lds = kMoeStreamLds * 2;
 #define QH_MOE(T, MD)                                                                                            \
   {                                                                                                              \
     static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(moe_stream_kernel<T, MD>),  \
