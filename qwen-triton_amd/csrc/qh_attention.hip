@@ -1397,15 +1397,18 @@ __global__ __launch_bounds__(256) void fa_decode_combine(const float* __restrict
   if (d == 0 && LSE) LSE[row] = L > 0.f ? (M + __log2f(L)) * kLn2 : -INFINITY;
 }
 
-// Decode for many sequences: one 256-thread workgroup per (b, kv-head) whose
-// wavefront w takes key tiles w, w + 4, w + 8, ... -- the key partition of
-// fa_decode_kernel with 4 interleaved splits, and the same per-tile arithmetic.
-// K fragments go from global memory straight into registers in the MFMA
-// operand layout (no LDS); V tiles go through two LDS stages per wavefront (the
-// transposed operand reads need LDS), so two workgroups fit on a CU. The four
-// partial (m, l, o) are combined in LDS in wavefront order with
-// fa_decode_combine's arithmetic: no workspace and no second launch, and the
-// same results as the split kernel plus combine at 4 splits.
+// Decode for many sequences: one workgroup of NW wavefronts per (b, kv-head) whose
+// wavefront w takes key tiles w, w + NW, w + 2 NW, ... with fa_decode_kernel's
+// per-tile arithmetic. K fragments go from global memory straight into registers
+// in the MFMA operand layout (no LDS); V tiles go through two LDS stages per
+// wavefront (the transposed operand reads need LDS), so two workgroups fit on a
+// CU. The partial (m, l, o) are combined in LDS in a fixed order with
+// fa_decode_combine's arithmetic: no workspace and no second launch. Up to
+// kDecodeTurnKeys keys a wavefront has one partial (with NW = 4 the results are
+// those of the split kernel plus combine at 4 splits); a longer stream is walked
+// from different parts on by different workgroups and has one partial per part
+// (below), so that a sequence's result depends on its own keys alone, not on its
+// place in the batch.
 //
 // K and V are __restrict__ except with PREP, where the kernel writes the new
 // cache rows and later reads them through the same pointers.
@@ -1422,6 +1425,10 @@ __global__ __launch_bounds__(256) void fa_decode_combine(const float* __restrict
 // tile's end (key p, and the rows past the last key that the tile load clamps
 // to it) are rewritten in the V stage. So no load waits for the stores, whose
 // bytes are those the patch supplies.
+// Keys up to which a stream is walked in order: nothing was gained by parting shorter ones (64 sequences of
+// 300 or 500 keys, four layers: 184 and 222 us either way).
+constexpr int kDecodeTurnKeys = 512;
+
 template <typename T, bool PREP>
 using kv_ptr = typename std::conditional<PREP, const T*, const T* __restrict__>::type;
 
@@ -1457,6 +1464,8 @@ __global__ __launch_bounds__(64 * NW) void fa_decode_wg_kernel(const T* __restri
                                                           const DecodePrepArgs<T, C> pa) {
   static_assert(G >= 1 && G <= 8, "query heads per kv-head");
   constexpr int BN = 32, NS = 2;
+  constexpr int NPART = G <= 4 ? 4 : 2;  // parts of a long stream, G of the 16 MFMA columns each
+  constexpr int NP = NPART * G;
   constexpr int CPR = DP / 8;    // 16-byte chunks per row
   constexpr int RPI = 64 / CPR;  // rows per 1 KiB load instruction
   constexpr int NI = BN / RPI;   // V load instructions per tile
@@ -1466,8 +1475,9 @@ __global__ __launch_bounds__(64 * NW) void fa_decode_wg_kernel(const T* __restri
   constexpr int KLD = 2 * KD;    // K load instructions per tile
   typedef typename Mfma<T>::v8 v8;
   __shared__ __attribute__((aligned(1024))) T Vs[NW][NS][BN * DP];
-  __shared__ float cml[NW][G][2];
-  __shared__ float co[NW][G][DP];
+  __shared__ float cml[NW][NP][2];
+  constexpr int COLD = DP + 4;  // floats per partial row: the rows of a store fall into different banks
+  static_assert(sizeof(Vs[0]) >= NP * COLD * sizeof(float), "a wavefront's partial outputs, over its V stages");
   __shared__ __attribute__((aligned(16))) T qs[PREP ? NW : 1][PREP ? G : 1][DP];
   __shared__ __attribute__((aligned(16))) T kvp[PREP ? NW : 1][2][PREP ? DP : 8];  // PREP: new key / value row
 
@@ -1482,17 +1492,31 @@ __global__ __launch_bounds__(64 * NW) void fa_decode_wg_kernel(const T* __restri
   const int sk_b = seqlens ? min(seqlens[b], Sk) : Sk;
   const int ntiles = w * BN < sk_b ? ((sk_b + BN - 1) / BN - w + NW - 1) / NW : 0;
 
-  // The wave's t-th tile: the workgroups walk their streams in lockstep, and where the distance
+  // The wave's t-th tile. The workgroups walk their streams in lockstep, and where the distance
   // between streams maps them onto few memory channels (caches of 2064, 2320, 1016 or 1032 positions,
-  // 512 bytes each) they take turns on those; starting a quarter of the stream apart by groups of 8
-  // workgroups keeps them spread. us per layer of a decode step, all from the start / quarters apart
-  // (64 sequences): 2064 positions 137 / 123, 2320 134 / 115, 1016 86 / 78; at other distances equal
-  // (2056: 110 / 110). 8 or 16 parts or pseudo-random starts cost 5-10 us at some power-of-two ones.
-  const int rot0 = ((bk >> 3) & 3) * ntiles >> 2;
-  auto tile_row = [&](int t) {
+  // 512 bytes each) they take turns on those; starting a part of the stream apart by groups of 8
+  // workgroups keeps them spread. us, four layers of a decode step (64 sequences), all from the start /
+  // parts apart: 2064 positions 542 / 483, 2320 585 / 499, 1016 331 / 306, 1032 343 / 317; at other
+  // distances equal (2056: 449 / 450, 4112: 765 / 769). 8 or 16 parts or pseudo-random starts cost 5-10 us a
+  // layer at some power-of-two distances; a start by kv-head alone is 506 at 2064.
+  // The softmax sums of part j stay in columns j G .. j G + G - 1 of the MFMA tiles, which hold the query
+  // rows once per part (16 columns, of which one part uses G): a tile's keys are hidden from the columns
+  // of the other parts, so the parts' sums do not depend on the order in which they are walked (0.4 us a
+  // layer, for the parts' combine).
+  const bool turn = sk_b > kDecodeTurnKeys;
+  int part0[NPART + 1];  // first tile of each part; short streams: one part
+#pragma unroll
+  for (int j = 0; j <= NPART; ++j) part0[j] = j == 0 ? 0 : (turn ? j * ntiles / NPART : ntiles);
+  int rot0 = 0;
+  if (turn)
+#pragma unroll
+    for (int j = 1; j < NPART; ++j)
+      if (((bk >> 3) & (NPART - 1)) == j) rot0 = part0[j];
+  auto tile_at = [&](int t) {
     const int tt = t + rot0;
-    return (w + (tt < ntiles ? tt : tt - ntiles) * NW) * BN;
+    return tt < ntiles ? tt : tt - ntiles;
   };
+  auto tile_row = [&](int t) { return (w + tile_at(t) * NW) * BN; };
 
   // K operand lanes: key 16 h + li of the tile, chunk d = 32 kd + 8 lg (clamped
   // into the row when D < DP; those products meet zero Q entries).
@@ -1611,7 +1635,7 @@ __global__ __launch_bounds__(64 * NW) void fa_decode_wg_kernel(const T* __restri
 #pragma unroll
     for (int kd = 0; kd < KD; ++kd) {
       const int d = kd * 32 + lg * 8;
-      if (li < G && d < D) qf[kd] = *reinterpret_cast<const v8*>(&qs[w][li][d]);
+      if (li < NP && d < D) qf[kd] = *reinterpret_cast<const v8*>(&qs[w][li % G][d]);
       else
 #pragma unroll
         for (int e = 0; e < 8; ++e) qf[kd][e] = (T)0.f;
@@ -1620,7 +1644,7 @@ __global__ __launch_bounds__(64 * NW) void fa_decode_wg_kernel(const T* __restri
 #pragma unroll
     for (int kd = 0; kd < KD; ++kd) {
       const int d = kd * 32 + lg * 8;
-      if (li < G && d < D) qf[kd] = *reinterpret_cast<const v8*>(Q + b * sqb + (int64_t)(hk * G + li) * sqh + d);
+      if (li < NP && d < D) qf[kd] = *reinterpret_cast<const v8*>(Q + b * sqb + (int64_t)(hk * G + li % G) * sqh + d);
       else
 #pragma unroll
         for (int e = 0; e < 8; ++e) qf[kd][e] = (T)0.f;
@@ -1641,12 +1665,16 @@ __global__ __launch_bounds__(64 * NW) void fa_decode_wg_kernel(const T* __restri
       s0 = mma16<T>(kf[0][kd], qf[kd], s0);
       s1 = mma16<T>(kf[1][kd], qf[kd], s1);
     }
-    const int kbase = tile_row(t) + 4 * lg;
+    const int tt = tile_at(t), kbase = (w + tt * NW) * BN + 4 * lg;
+    int part = 0;
+#pragma unroll
+    for (int j = 1; j < NPART; ++j) part += tt >= part0[j];
+    const int kend = li / G == part ? sk_b : 0;  // keys that this column sees
     float x[8];
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      x[r] = kbase + r < sk_b ? s0[r] * scale_log2 : -INFINITY;
-      x[4 + r] = kbase + 16 + r < sk_b ? s1[r] * scale_log2 : -INFINITY;
+      x[r] = kbase + r < kend ? s0[r] * scale_log2 : -INFINITY;
+      x[4 + r] = kbase + 16 + r < kend ? s1[r] * scale_log2 : -INFINITY;
     }
     float mx = fmaxf(fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3])), fmaxf(fmaxf(x[4], x[5]), fmaxf(x[6], x[7])));
     mx = fmaxf(mx, __shfl_xor(mx, 16));
@@ -1726,35 +1754,40 @@ __global__ __launch_bounds__(64 * NW) void fa_decode_wg_kernel(const T* __restri
   }
   l += __shfl_xor(l, 16);
   l += __shfl_xor(l, 32);
-  if (li < G) {
+  if (li < NP) {
+    float* co = reinterpret_cast<float*>(&Vs[w][0][0]) + li * COLD + 4 * lg;  // (the wave has read its V stages)
 #pragma unroll
-    for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) co[w][li][dt * 16 + 4 * lg + r] = o[dt][r];
+    for (int dt = 0; dt < DT; ++dt) *reinterpret_cast<f32x4*>(co + dt * 16) = o[dt];
     if (lg == 0) {
       cml[w][li][0] = m;
       cml[w][li][1] = l;
     }
   }
   __syncthreads();
-  // combine the four wavefronts in order (fa_decode_combine's arithmetic)
-  for (int idx = threadIdx.x; idx < G * DP; idx += 64 * NW) {
-    const int g = idx / DP, d = idx % DP;
-    float M = -INFINITY;
+  // combine the wavefronts' parts in order (fa_decode_combine's arithmetic; a part without keys adds 0)
+  auto combine = [&](auto parts) {
+    constexpr int P = decltype(parts)::value;
+    for (int idx = threadIdx.x; idx < G * DP; idx += 64 * NW) {
+      const int g = idx / DP, d = idx % DP;
+      float M = -INFINITY;
 #pragma unroll
-    for (int s = 0; s < NW; ++s) M = fmaxf(M, cml[s][g][0]);
-    const float Mr = (M == -INFINITY) ? 0.f : M;
-    float L = 0.f, acc = 0.f;
+      for (int s = 0; s < NW * P; ++s) M = fmaxf(M, cml[s / P][s % P * G + g][0]);
+      const float Mr = (M == -INFINITY) ? 0.f : M;
+      float L = 0.f, acc = 0.f;
 #pragma unroll
-    for (int s = 0; s < NW; ++s) {
-      const float wgt = exp2_(cml[s][g][0] - Mr);
-      L += cml[s][g][1] * wgt;
-      acc += co[s][g][d] * wgt;
+      for (int s = 0; s < NW * P; ++s) {
+        const int c = s % P * G + g;
+        const float wgt = exp2_(cml[s / P][c][0] - Mr);
+        L += cml[s / P][c][1] * wgt;
+        acc += reinterpret_cast<const float*>(&Vs[s / P][0][0])[c * COLD + d] * wgt;
+      }
+      const int64_t row = (int64_t)bk * G + g;
+      if (d < D) O[row * D + d] = from_f32<T>(L > 0.f ? acc / L : 0.f);
+      if (d == 0 && LSE) LSE[row] = L > 0.f ? (M + __log2f(L)) * kLn2 : -INFINITY;
     }
-    const int64_t row = (int64_t)bk * G + g;
-    if (d < D) O[row * D + d] = from_f32<T>(L > 0.f ? acc / L : 0.f);
-    if (d == 0 && LSE) LSE[row] = L > 0.f ? (M + __log2f(L)) * kLn2 : -INFINITY;
-  }
+  };
+  if (turn) combine(std::integral_constant<int, NPART>{});
+  else combine(std::integral_constant<int, 1>{});
 }
 
 static int pick_dp(int64_t D) {

@@ -510,3 +510,49 @@ def test_moe_tokens_on_few_experts_are_not_streamed_twice():
         return min(times)
 
     assert best(128) <= 1.3 * best(8)
+
+
+# One workgroup per (sequence, kv-head) starts long streams at different parts: a sequence's result may not
+# depend on its place in the batch (equal sequences in slots of every starting part), and it is right where
+# parts hold no tile, one or many; lengths on both sides of the 512 keys up to which a stream is not parted.
+@pytest.mark.parametrize("Hq,Hkv", [(8, 8), (16, 8), (32, 8), (64, 8)])
+@pytest.mark.parametrize("Sk", [513, 640, 1111, 2050])
+def test_decode_attention_does_not_depend_on_the_slot(Hq, Hkv, Sk):
+    from qwen_triton.kernels.flash_attention import flash_decode
+
+    n, reps, D, dt = 6, 11, 128, torch.bfloat16  # 6 sequences, each in 11 slots
+    q, k, v = (_rand(n, h, s, D, dtype=dt, seed=i) for i, (h, s) in enumerate([(Hq, 1), (Hkv, Sk), (Hkv, Sk)]))
+    lens = torch.tensor([Sk, 512, 513, Sk - 1, 33, (Sk + 513) // 2], dtype=torch.int32).clamp(max=Sk)
+    slot = torch.arange(n * reps) % n
+    i = slot.cuda()
+    out = flash_decode(q[i], k[i].contiguous(), v[i].contiguous(), D ** -0.5, Hq // Hkv, seqlens=lens[slot].cuda())
+    assert torch.equal(out, out[:n][i])
+    qd, kd, vd = (t.cpu().double() for t in (q, k, v))
+    kd, vd = (t.repeat_interleave(Hq // Hkv, dim=1) for t in (kd, vd))
+    s = torch.matmul(qd, kd.transpose(2, 3)) * D ** -0.5
+    s = s.masked_fill(torch.arange(Sk)[None, None, None, :] >= lens[:, None, None, None], float("-inf"))
+    p = torch.softmax(s, -1)
+    ref = torch.matmul(p, vd)
+    # probabilities and outputs are rounded to bf16 once each
+    bound = EPS[dt] * (torch.matmul(p, vd.abs()) + ref.abs()) + 1e-6
+    assert ((out[:n].cpu().double() - ref).abs() <= bound).all()
+
+
+# The step that prepares its own rows: the same, for 8 wavefronts (32 sequences) and 4.
+@pytest.mark.parametrize("B,Sk,pos", [(32, 1100, 1099), (32, 520, 100), (72, 2050, 1300)])
+def test_decode_step_does_not_depend_on_the_slot(B, Sk, pos):
+    from qwen_triton import _native
+
+    Hq, Hkv, D, dt, n = 16, 8, 128, torch.bfloat16, 4
+    i = torch.arange(B, device="cuda") % n
+    q2, k2, v2 = (_rand(n, h * D, dtype=dt, seed=j)[i] for j, h in enumerate((Hq, Hkv, Hkv)))
+    wq, wk = (_rand(D, dtype=dt, seed=5 + j) for j in range(2))
+    cos, sin = (torch.full((1, 1, D), c, dtype=dt, device="cuda") for c in (0.8, 0.6))
+    kc, vc = (_rand(n, Hkv, Sk, D, dtype=dt, seed=9 + j)[i].contiguous() for j in range(2))
+    out = torch.empty(B, Hq, D, dtype=dt, device="cuda")
+    p, code = torch.tensor([pos], device="cuda"), _native.dtype_code(dt)
+    _native.call("qh_flash_decode_prepare", q2.data_ptr(), Hq * D, k2.data_ptr(), Hkv * D, v2.data_ptr(), Hkv * D,
+                 wq.data_ptr(), wk.data_ptr(), 1e-6, 0, cos.data_ptr(), sin.data_ptr(), D, 1, D, kc.data_ptr(),
+                 *kc.stride()[:3], vc.data_ptr(), *vc.stride()[:3], Sk, p.data_ptr(), out.data_ptr(), None, None, B, Hq,
+                 Hkv, Sk, D, D ** -0.5, code, code, code, _native.stream(out.device))
+    assert torch.equal(out, out[:n][i]) and torch.equal(kc, kc[:n][i])
