@@ -339,14 +339,14 @@ int qh_gemm_multi_rms(int64_t M, int64_t K, const void* A, int64_t lda, int coun
 /* Up to three products of more than 128 rows that share A (row-major, k-contiguous), in one launch:
  * C_i = A B_i^T (+ bias_i), or gated (two products of equal N, a multiple of 64, no bias)
  * C_0 = silu(C_gate) * C_up with each product rounded to the dtype first. Host arrays of count
- * entries. Shapes with qh_gemm_group_ok() != 0; every output equals the separate qh_gemm's bit for bit
+ * entries. Shapes with qh_gemm_group_ok() != 0; every output equals the separate qh_gemm_ws's bit for bit
  * (gated: qh_silu_mul_fwd's of those, in fp16 to one unit in the last place). bf16/f16; A, B_i 16-byte
  * aligned with K, lda, ldb multiples of 8, lda and ldb below 2^27 elements (else QH_E_ARG).
  * Replaces, fused, the same reference calls as qh_gemm_multi for prompts past its 128 rows. */
 int qh_gemm_group(int64_t M, int64_t K, const void* A, int64_t lda, int count, const void* const* B,
                   const int64_t* ldb, const int64_t* N, void* const* C, const int64_t* ldc,
                   const void* const* bias, int gated, int dtype, void* stream);
-int64_t qh_gemm_group_ok(int64_t M, int count, const int64_t* N, int gated);
+int64_t qh_gemm_group_ok(int64_t M, int64_t K, int count, const int64_t* N, int gated);
 /* out[n] = sum_m X[m*ldx + n] in a fixed order (bias gradient).
  * Replaces qwen_triton/kernels/matmul.py:114-127 (_row_sum_kernel). */
 int qh_colsum(const void* X, int64_t ldx, int64_t M, int64_t N, void* out, int dtype, int out_dtype,

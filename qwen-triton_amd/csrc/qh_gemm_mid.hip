@@ -2,6 +2,7 @@
 // qh_gemm_mid.h); bf16 products. The other types are in qh_gemm_mid_f16.hip.
 #include "qh_gemm_mid_run.h"
 
+int qh_gemm_splitk_count(int64_t M, int64_t N, int64_t K);
 int qh_gemm_mid_f16(int v, int ta, int tb, int M, int N, int K, const void* A, int64_t lda, const void* B, int64_t ldb,
                     void* C, int64_t ldc, const void* bias, int out_dtype, hipStream_t st);
 
@@ -36,14 +37,16 @@ int qh_gemm_mid_dispatch(int ta, int tb, int M, int N, int K, const void* A, int
 // Several products of 128 to about 1000 rows that share A (q/k/v; gate/up with SiLU-mul), one launch.
 // All of the tiles it uses, and those the products take on their own where it is taken, split k over
 // two wave groups in the same way, so each output has the bits of the separate products: a product
-// that would go to a tile with another split keeps its own launch. 0: not taken, else the tile.
-static int group_pick(int64_t M, int count, const int64_t* N, bool gated) {
+// that would go to a tile with another split, or whose K would be split over workgroups, keeps its own
+// launch. 0: not taken, else the tile.
+static int group_pick(int64_t M, int64_t K, int count, const int64_t* N, bool gated) {
   if (M <= 128 || count < 2 || count > kMidProducts) return 0;
   int64_t t64 = 0, t64128 = 0, t128 = 0;
   for (int i = 0; i < count; ++i) {
     if (N[i] <= 0 || N[i] >= (1ll << 31)) return 0;
     const int v = mid_pick(M, N[i]);
     if (v != MID_64x64 && v != MID_64x128 && v != MID_128x128) return 0;
+    if (qh_gemm_splitk_count(M, N[i], K) > 1) return 0;
     t64 += ((M + 63) / 64) * ((N[i] + 63) / 64);
     t64128 += ((M + 63) / 64) * ((N[i] + 127) / 128);
     t128 += ((M + 127) / 128) * ((N[i] + 127) / 128);
@@ -54,8 +57,8 @@ static int group_pick(int64_t M, int count, const int64_t* N, bool gated) {
   return t128 <= 256 ? MID_128x128 : 0;
 }
 
-extern "C" int64_t qh_gemm_group_ok(int64_t M, int count, const int64_t* N, int gated) {
-  return group_pick(M, count, N, gated != 0) > 0;
+extern "C" int64_t qh_gemm_group_ok(int64_t M, int64_t K, int count, const int64_t* N, int gated) {
+  return group_pick(M, K, count, N, gated != 0) > 0;
 }
 
 template <typename T>
@@ -90,7 +93,7 @@ extern "C" int qh_gemm_group(int64_t M, int64_t K, const void* A, int64_t lda, i
                              const int64_t* ldb, const int64_t* N, void* const* C, const int64_t* ldc,
                              const void* const* bias, int gated, int dtype, void* stream) {
   QH_CHECK_ARG(K > 0 && K < (1ll << 31) && M < (1ll << 31), "qh_gemm_group: bad shape");
-  const int v = group_pick(M, count, N, gated != 0);
+  const int v = group_pick(M, K, count, N, gated != 0);
   QH_CHECK_ARG(v > 0, "qh_gemm_group: shape not served (see qh_gemm_group_ok)");
   QH_CHECK_ARG(dtype == QH_BF16 || dtype == QH_F16, "qh_gemm_group: bf16/f16 only");
   QH_CHECK_ARG(aligned16(A) && lda % 8 == 0 && lda >= K && K % 8 == 0,

@@ -108,7 +108,7 @@ def linear_group_rows_ok(x: torch.Tensor, weights: list[torch.Tensor],
     rows = _rows(x, k)  # (a view unless the rows have to be copied for any product)
     if rows.stride(0) % 8 or rows.stride(0) >= _GROUP_MAX_STRIDE or rows.data_ptr() % 16:
         return False
-    return bool(_native.call("qh_gemm_group_ok", rows.shape[0], len(weights),
+    return bool(_native.call("qh_gemm_group_ok", rows.shape[0], k, len(weights),
                              ctypes.addressof(_group_plan(weights, biases)[2]), int(gated)))
 
 

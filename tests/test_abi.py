@@ -131,3 +131,11 @@ def test_fused_loss_refuses_rows_past_its_lane_offsets(ldx, ldw):
     with pytest.raises(_native.NativeUnsupported, match="elements apart"):
         _native.call("qh_lmce_rows_fwd", 4096, ldx, 4096, ldw, 4096, 512, 1024, 64, -100, 4096, 1024, 4096, 4096,
                      4096, 1 << 30, _native.BF16, 0)
+
+
+def test_grouped_products_leave_split_k_alone():
+    n = (ctypes.c_int64 * 2)(3072, 3072)
+    ok = lambda K: _native.call("qh_gemm_group_ok", 517, K, 2, ctypes.addressof(n), 1)  # noqa: E731
+    assert ok(1024) and ok(8184) and not ok(8192)
+    assert not _native.call("qh_gemm_workspace", 517, 3072, 8184, _native.BF16)
+    assert _native.call("qh_gemm_workspace", 517, 3072, 8192, _native.BF16)

@@ -240,6 +240,24 @@ def test_gemm_group_equals_the_separate_products(M, ns, K, dtype):
                 assert ((got.double() - want.double()).abs() <= 2.0 ** -10 * want.double().abs() + 2.0 ** -24).all()
 
 
+# From K = 8192 on the separate products split K over workgroups: they keep their launches, and their bits.
+@pytest.mark.parametrize("K", [8184, 8192])
+def test_gemm_group_leaves_split_products_alone(K):
+    from qwen_triton import kernels
+    from qwen_triton.modules import QwenMLP
+
+    dt = torch.bfloat16
+    torch.manual_seed(0)
+    mlp = QwenMLP(K, 1536).to("cuda", dt).eval()
+    x = _rand(1, 517, K, dtype=dt, seed=1)
+    seen = []
+    mlp.down_proj.register_forward_pre_hook(lambda m, a: seen.append(a[0]))
+    with torch.no_grad():
+        mlp(x)
+        want = kernels.silu_mul(mlp.gate_proj(x), mlp.up_proj(x))
+    assert torch.equal(seen[0], want)
+
+
 # A prompt past 128 rows calls a projection module that does more than its product (a forward hook, a
 # replaced forward), and its result is used.
 @pytest.mark.parametrize("how", ["hook", "pre_hook", "forward"])
