@@ -59,7 +59,9 @@ def gemm(trans_a: bool, trans_b: bool, M: int, N: int, K: int, a: torch.Tensor, 
     code = _native.dtype_code(a.dtype)
     args = (int(trans_a), int(trans_b), M, N, K, a.data_ptr(), lda, b.data_ptr(), ldb, out.data_ptr(), ldc,
             None if bias is None else bias.data_ptr(), code, _native.dtype_code(out.dtype))
-    if K >= 8192 and N >= 256 and M * N < 128 * 65536:
+    # (decode products, both operands k-contiguous, split K inside their workgroups)
+    decode = M <= 128 and not (M > 16 and N > 8192) and not trans_a and not trans_b
+    if K >= 8192 and N >= 256 and M * N < 128 * 65536 and not decode:
         nbytes = _native.call("qh_gemm_workspace", M, N, K, code)
         if nbytes:
             ws = _native.workspace(nbytes, a.device)

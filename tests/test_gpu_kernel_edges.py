@@ -43,6 +43,24 @@ def test_gemm_tile_choice_and_remainders(M, N, K, ta, tb, dtype, out_dtype):
     assert (out[:, N:] == 7.0).all()
 
 
+def test_gemm_asks_for_no_workspace_that_its_kernel_does_not_take():
+    """Decode products (up to 128 rows, both operands k-contiguous) run in one launch whatever K is."""
+    from qwen_triton import _native, kernels
+
+    dt = torch.bfloat16
+    x, w = _rand(64, 16384, dtype=dt, seed=1), _rand(512, 16384, dtype=dt, seed=2, scale=0.02)
+    with torch.no_grad():
+        kernels.triton_matmul(x, w)
+        torch.cuda.synchronize()
+        calls, used = _native.CALLS["qh_gemm_ws"], torch.cuda.memory_allocated()
+        torch.cuda.reset_peak_memory_stats()
+        out = kernels.triton_matmul(x, w)
+    assert _native.CALLS["qh_gemm_ws"] == calls
+    assert torch.cuda.max_memory_allocated() - used <= out.numel() * 2 + 512
+    ref = x.cpu().double() @ w.cpu().double().T
+    assert ((out.cpu().double() - ref).abs() <= 2 * EPS[dt] * ref.abs() + 1e-3).all()
+
+
 def _delta_inputs(B, S, H, K, V, seed, initial):
     import torch.nn.functional as F
 
