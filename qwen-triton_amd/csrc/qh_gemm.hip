@@ -19,6 +19,7 @@
 //    wavefront per output column.
 #include "qh_mfma.h"
 #include "qh_lds.h"
+#include "qh_lds_limit.h"
 
 // Large-tile and split-K paths (qh_gemm_tile.hip).
 int qh_gemm_tile_dispatch(int ta, int tb, int M, int N, int K, const void* A, int64_t lda, const void* B,
@@ -1372,9 +1373,9 @@ extern "C" int qh_moe_gemm(int mode, const void* A, int64_t lda, const int32_t* 
     constexpr int lds = kMoeStreamLds * 2;
 #define QH_MOE(T, MD)                                                                                            \
   {                                                                                                              \
-    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(moe_stream_kernel<T, MD>),  \
-                                                       hipFuncAttributeMaxDynamicSharedMemorySize, lds);         \
-    QH_CHECK_HIP(attr, "qh_moe_gemm: LDS attribute");                                                            \
+    static qh::LdsLimit limit;                                                                                   \
+    if (const int rc = limit.raise(reinterpret_cast<const void*>(moe_stream_kernel<T, MD>), lds, "qh_moe_gemm")) \
+      return rc;                                                                                                 \
     moe_stream_kernel<T, MD><<<grid, 256, lds, st>>>((const T*)A, lda, rows, (const T* const*)B_table, ldb,      \
                                                      (T*)C, ldc, (const T*)wrow, seg_off, tile_off, (int)E,      \
                                                      (int)N, (int)K);                                            \

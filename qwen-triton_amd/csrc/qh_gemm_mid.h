@@ -28,6 +28,7 @@
 // 439 -> 36, 384x3072x1024 193 -> 33, its weight gradient 79 -> 29 (83 of 157 TFLOP/s).
 #pragma once
 
+#include "qh_lds_limit.h"
 #include "qh_tile_layout.h"
 
 namespace {
@@ -244,12 +245,8 @@ int mid_run(const T* A, int64_t lda, const T* B, int64_t ldb, OT* C, int64_t ldc
   constexpr int lds = WK * NS * (BM + BN) * 128;
   static_assert(lds <= 160 * 1024, "LDS");
   auto* kern = gemm_mid_kernel<T, OT, BM, BN, WM, WN, WK, NS, AT, BT>;
-  static const hipError_t attr =
-      hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-  if (attr != hipSuccess) {
-    qh::set_error("qh_gemm: LDS attribute: %s", hipGetErrorString(attr));
-    return QH_E_HIP;
-  }
+  static qh::LdsLimit limit;
+  if (const int rc = limit.raise(reinterpret_cast<const void*>(kern), lds, "qh_gemm")) return rc;
   const int tm = (M + BM - 1) / BM, tn = (N + BN - 1) / BN;
   kern<<<(unsigned)(tm * tn), 64 * WM * WN * WK, lds, st>>>(A, lda, B, ldb, C, ldc, bias, M, N, K, tm, tn, MidGroup<T>{});
   return QH_OK;
@@ -259,12 +256,8 @@ template <typename T, int BM, int BN, int WK, int NS, int MODE>
 int mid_group_run(const T* A, int64_t lda, const MidGroup<T>& grp, int M, int K, int tiles_n, hipStream_t st) {
   constexpr int lds = WK * NS * (BM + BN) * 128;
   auto* kern = gemm_mid_kernel<T, T, BM, BN, 2, 2, WK, NS, false, false, MODE>;
-  static const hipError_t attr =
-      hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-  if (attr != hipSuccess) {
-    qh::set_error("qh_gemm_group: LDS attribute: %s", hipGetErrorString(attr));
-    return QH_E_HIP;
-  }
+  static qh::LdsLimit limit;
+  if (const int rc = limit.raise(reinterpret_cast<const void*>(kern), lds, "qh_gemm_group")) return rc;
   const int tm = (M + BM - 1) / BM;
   kern<<<(unsigned)(tm * tiles_n), 64 * 4 * WK, lds, st>>>(A, lda, grp.B[0], grp.ldb[0], grp.C[0], grp.ldc[0], nullptr,
                                                            M, grp.N[0], K, tm, tiles_n, grp);

@@ -3,6 +3,8 @@ from __future__ import annotations
 
 import ctypes
 import re
+import shutil
+import subprocess
 import warnings
 from pathlib import Path
 
@@ -139,3 +141,48 @@ def test_grouped_products_leave_split_k_alone():
     assert ok(1024) and ok(8184) and not ok(8192)
     assert not _native.call("qh_gemm_workspace", 517, 3072, 8184, _native.BF16)
     assert _native.call("qh_gemm_workspace", 517, 3072, 8192, _native.BF16)
+
+
+_LDS_LIMIT_PROGRAM = r"""
+#include "qh_lds_limit.h"
+#include <cstdio>
+static int device = 0, calls = 0, failures = 0;
+extern "C" hipError_t hipGetDevice(int* d) { *d = device; return hipSuccess; }
+extern "C" hipError_t hipFuncSetAttribute(const void*, hipFuncAttribute, int) {
+  ++calls;
+  return failures-- > 0 ? hipErrorUnknown : hipSuccess;
+}
+extern "C" const char* hipGetErrorString(hipError_t) { return "injected"; }
+namespace qh { void set_error(const char*, ...) {} }
+int main() {
+  static qh::LdsLimit limit;
+  failures = 1;
+  const int first = limit.raise("k", 1 << 17, "t");  // the attribute call fails: reported, not remembered
+  for (int i = 0; i < 3; ++i)
+    if (limit.raise("k", 1 << 17, "t") != QH_OK) return 1;
+  const int on0 = calls;
+  device = 1;
+  for (int i = 0; i < 3; ++i)
+    if (limit.raise("k", 1 << 17, "t") != QH_OK) return 1;
+  device = 64;
+  std::printf("%d %d %d %d", first != QH_OK, on0, calls, limit.raise("k", 1 << 17, "t") != QH_OK);
+  return 0;
+}
+"""
+
+
+def test_lds_limit_is_raised_on_every_device(tmp_path):
+    """A kernel's dynamic LDS limit belongs to a device: every place that raises it looks at the current
+    one, and the helper sets it once on each and again after a failure."""
+    csrc = ROOT / "qwen-triton_amd" / "csrc"
+    for f in [*csrc.glob("*.h"), *csrc.glob("*.hip")]:
+        assert ("hipFuncSetAttribute" in f.read_text()) <= ("hipGetDevice" in f.read_text()), f.name
+    if shutil.which("hipcc") is None and not Path("/opt/rocm/bin/hipcc").exists():
+        pytest.skip("no hipcc")
+    (tmp_path / "t.cpp").write_text(_LDS_LIMIT_PROGRAM)
+    exe = tmp_path / "t"
+    subprocess.run([shutil.which("hipcc") or "/opt/rocm/bin/hipcc", "-x", "hip", "--offload-host-only", "-std=c++17", "-fPIE",
+                    f"-I{csrc}", f"-I{ROOT / 'include'}", "-c", str(tmp_path / "t.cpp"), "-o", str(tmp_path / "t.o")],
+                   check=True)
+    subprocess.run(["g++", str(tmp_path / "t.o"), "-o", str(exe)], check=True)
+    assert subprocess.run([str(exe)], check=True, capture_output=True, text=True).stdout == "1 2 3 1"
