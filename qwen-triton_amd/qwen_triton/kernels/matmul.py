@@ -42,6 +42,15 @@ def _torch_matmul_backward(x, weight, grad_output, needs_bias_grad: bool):
     return grad_x, grad_weight, grad_bias
 
 
+def _rows_view(t: torch.Tensor, cols: int) -> torch.Tensor | None:
+    """2-D row-major view [rows, cols] with unit column stride; None where there is none."""
+    try:
+        t2 = t.view(-1, cols)
+    except RuntimeError:
+        return None
+    return None if t2.stride(1) != 1 or (t2.shape[0] > 1 and t2.stride(0) < cols) else t2
+
+
 def _rows(t: torch.Tensor, cols: int) -> torch.Tensor:
     """2-D row-major view [rows, cols] with unit column stride (copies only if needed)."""
     t2 = t.reshape(-1, cols)
@@ -107,10 +116,10 @@ def linear_group_rows_ok(x: torch.Tensor, weights: list[torch.Tensor],
         return False
     if gated and weights[0].stride(0) != weights[1].stride(0):
         return False
-    rows = _rows(x, k)  # (a view unless the rows have to be copied for any product)
-    if rows.stride(0) % 8 or rows.stride(0) >= _GROUP_MAX_STRIDE or rows.data_ptr() % 16:
+    rows = _rows_view(x, k)  # (None: copied for any product, to aligned contiguous rows)
+    if rows is not None and (rows.stride(0) % 8 or rows.stride(0) >= _GROUP_MAX_STRIDE or rows.data_ptr() % 16):
         return False
-    return bool(_native.call("qh_gemm_group_ok", rows.shape[0], k, len(weights),
+    return bool(_native.call("qh_gemm_group_ok", n // k, k, len(weights),
                              ctypes.addressof(_group_plan(weights, biases)[2]), int(gated)))
 
 

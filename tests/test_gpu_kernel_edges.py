@@ -258,6 +258,27 @@ def test_gemm_group_equals_the_separate_products(M, ns, K, dtype):
                 assert ((got.double() - want.double()).abs() <= 2.0 ** -10 * want.double().abs() + 2.0 ** -24).all()
 
 
+# Rows that a product has to copy first are not copied to look at them.
+@pytest.mark.parametrize("form", ["every_other", "overlapping", "expanded", "plain"])
+def test_grouped_rows_are_not_copied_to_look_at_them(form):
+    from qwen_triton import kernels
+    from qwen_triton.kernels.matmul import linear_group, linear_group_rows_ok
+
+    M, K, dt = 300, 256, torch.bfloat16
+    base = _rand(M * 2 * K, dtype=dt, seed=1)
+    x = dict(every_other=base.view(M, 2 * K)[:, ::2], overlapping=base.as_strided((M, K), (8, 1)),
+             expanded=base[:K].expand(2, M // 2, K), plain=base.view(M, 2 * K)[:, :K])[form]
+    ws = [_rand(n, K, dtype=dt, seed=2 + i, scale=0.1) for i, n in enumerate((2048, 2056))]
+    with torch.no_grad():
+        linear_group_rows_ok(x, ws)
+        count = lambda: torch.cuda.memory_stats()["allocation.all.allocated"]  # noqa: E731
+        before = count()
+        assert linear_group_rows_ok(x, ws)
+        assert count() == before
+        for w, o in zip(ws, linear_group(x, ws)):
+            assert torch.equal(o, kernels.triton_matmul(x, w))
+
+
 # From K = 8192 on the separate products split K over workgroups: they keep their launches, and their bits.
 @pytest.mark.parametrize("K", [8184, 8192])
 def test_gemm_group_leaves_split_products_alone(K):
