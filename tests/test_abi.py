@@ -182,7 +182,7 @@ def test_lds_limit_is_raised_on_every_device(tmp_path):
     (tmp_path / "t.cpp").write_text(_LDS_LIMIT_PROGRAM)
     exe = tmp_path / "t"
     hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
-    subprocess.run([hipcc, "-x", "hip", "--offload-host-only", "-std=c++17", "-fPIE", f"-I{csrc}", f"-I{ROOT / 'include'}", "-c", str(tmp_path / "t.cpp"), "-o", str(tmp_path / "t.o")],
-                   check=True)
+    subprocess.run([hipcc, "-x", "hip", "--offload-host-only", "-std=c++17", "-fPIE", f"-I{csrc}",
+                    f"-I{ROOT / 'include'}", "-c", str(tmp_path / "t.cpp"), "-o", str(tmp_path / "t.o")], check=True)
     subprocess.run(["g++", str(tmp_path / "t.o"), "-o", str(exe)], check=True)
     assert subprocess.run([str(exe)], check=True, capture_output=True, text=True).stdout == "1 2 3 1"

@@ -106,6 +106,35 @@ def test_delta_rule_chunks(S, K, V, initial):
     assert err(st.cpu()) <= 1.25 * err(_delta_reference(*args, torch.float32)[1])
 
 
+# Keys with a common direction, of norm 1 (solved in chunks) and beyond (chunks whose update is no contraction
+# run token by token), a call with both, and growing states (positive log-decays).
+@pytest.mark.parametrize("K,V", [(128, 72), (64, 64)])
+@pytest.mark.parametrize("norm,cosine,growth", [(1.0, 0.9, False), (1.4, 0.9, False), (1.6, 0.99, False),
+                                                (2.0, 0.0, False), ("rising", 0.9, False), (1.0, 0.9, True)])
+def test_delta_rule_chunks_of_related_keys(K, V, norm, cosine, growth):
+    import torch.nn.functional as F
+
+    from qwen_triton.kernels import gated_delta_rule_sequence
+
+    q, k, v, decay, beta, state = _delta_inputs(1, 400, 3, K, V, 61, True)
+    g = torch.Generator().manual_seed(62)
+    common = F.normalize(torch.randn(1, 1, 3, K, generator=g), dim=-1)
+    size = torch.linspace(1.0, 1.5, 400)[None, :, None, None] if norm == "rising" else norm
+    k = (F.normalize(cosine ** 0.5 * common + (1 - cosine) ** 0.5 * k.float(), dim=-1) * size).bfloat16()
+    beta = torch.sigmoid(2 + torch.randn(1, 400, 3, generator=g))
+    decay = torch.full_like(decay, 0.01) if growth else decay * 0.3
+    args = (q, k, v, decay, beta, state)
+    out, st = gated_delta_rule_sequence(*(t.cuda() for t in args[:5]), initial_state=state.cuda())
+    ro, rs = _delta_reference(*args, torch.float64)
+    fo, fs = _delta_reference(*args, torch.float32)
+    err = lambda x, r: float((x.double() - r).norm() / r.norm())  # noqa: E731
+    # the state is as close to fp64 as the recurrence in fp32 (a quarter for another order of the sums);
+    # solved chunks of related keys up to twice as far: their corrections are as large as the values
+    solved = norm == 1.0 or norm == "rising"
+    assert err(st.cpu(), rs) <= (2.0 if solved else 1.25) * err(fs, rs)
+    assert err(out.cpu(), ro) <= EPS[torch.bfloat16] + 2 * err(fo, ro)
+
+
 def test_delta_rule_split_at_a_chunk_boundary():
     """Two launches through the state, split at a multiple of 64 tokens: the bits of one launch."""
     from qwen_triton.kernels import gated_delta_rule_sequence as rule
