@@ -136,7 +136,7 @@ def test_delta_rule_chunks_of_related_keys(K, V, norm, cosine, growth):
 
 
 def test_delta_rule_split_at_a_chunk_boundary():
-    """Two launches through the state, split at a multiple of 64 tokens: the bits of one launch."""
+    """Two launches of at least 320 tokens, split at a multiple of 64: the bits of one launch."""
     from qwen_triton.kernels import gated_delta_rule_sequence as rule
 
     q, k, v, g, b, s0 = (t.cuda() for t in _delta_inputs(1, 750, 2, 128, 128, 5, True))
@@ -144,6 +144,23 @@ def test_delta_rule_split_at_a_chunk_boundary():
     o1, s1 = rule(*(t[:, :384] for t in (q, k, v, g, b)), initial_state=s0)
     o2, s2 = rule(*(t[:, 384:] for t in (q, k, v, g, b)), initial_state=s1)
     assert torch.equal(torch.cat((o1, o2), 1), out) and torch.equal(s2, st)
+
+
+@pytest.mark.parametrize("S,first", [(384, 320), (448, 64), (401, 400), (700, 350)])
+def test_delta_rule_continued_by_a_call_of_another_kind(S, first):
+    """A call of fewer than 320 tokens runs token by token, and a split off the 64-token grid moves the chunks:
+    two calls through the state are then as close to 64 bits as one, not equal to it in every bit."""
+    from qwen_triton.kernels import gated_delta_rule_sequence as rule
+
+    args = _delta_inputs(1, S, 2, 128, 64, 9, True)
+    q, k, v, g, b, s0 = (t.cuda() for t in args)
+    o1, s1 = rule(*(t[:, :first] for t in (q, k, v, g, b)), initial_state=s0)
+    o2, s2 = rule(*(t[:, first:] for t in (q, k, v, g, b)), initial_state=s1)
+    ro, rs = _delta_reference(*args, torch.float64)
+    err = lambda x: float((x.double() - rs).norm() / rs.norm())  # noqa: E731
+    assert err(s2.cpu()) <= 1.25 * err(_delta_reference(*args, torch.float32)[1])
+    out = torch.cat((o1, o2), 1).cpu().double()
+    assert ((out - ro).abs() <= EPS[torch.bfloat16] * ro.abs() + 2e-6).all()
 
 
 @pytest.mark.parametrize("case", ["nan_value", "inf_value", "nan_key", "reset", "reset_all"])
@@ -278,7 +295,10 @@ def test_gemm_group_equals_the_separate_products(M, ns, K, dtype):
                 assert torch.equal(o, kernels.triton_matmul(x, w, b))
         n = ns[0] // 64 * 64
         gu = [ws[0][:n], _rand(n, K, dtype=dtype, seed=20, scale=0.1)]
-        if linear_group_rows_ok(x, gu, gated=True):
+        # (517, 1024): 64x128 tiles; (517, 2048) and (1000, 2048): 128x128
+        gated = linear_group_rows_ok(x, gu, gated=True)
+        assert gated == (-(-M // 32) * (n // 64) > 256)
+        if gated:
             want = kernels.silu_mul(kernels.triton_matmul(x, gu[0]), kernels.triton_matmul(x, gu[1]))
             got = linear_group(x, gu, gated=True)
             if dtype == torch.bfloat16:
