@@ -158,6 +158,17 @@ def ptr(t: torch.Tensor | None) -> int | None:
     return None if t is None else t.data_ptr()
 
 
+_functorch_level, _dispatch_modes = torch._C._functorch.peek_interpreter_stack, torch._C._len_torch_dispatch_stack
+_FAKE_MODE = torch._C._TorchDispatchModeKey.FAKE
+
+
+def in_transform() -> bool:
+    """True inside a functorch transform (vmap, jvp, functionalize, ...) or a FakeTensorMode: tensors
+    there stand for others and have no memory to hand to a kernel (``data_ptr()`` raises or is 0)."""
+    return _functorch_level() is not None or (
+        _dispatch_modes() > 0 and torch._C._get_dispatch_mode(_FAKE_MODE) is not None)
+
+
 def stream(device: torch.device | None = None) -> int:
     """Raw handle of torch's current stream on ``device`` (the stream every kernel is enqueued on)."""
     if device is None:

@@ -105,7 +105,7 @@ def linear_group_rows_ok(x: torch.Tensor, weights: list[torch.Tensor],
     if n <= 128 * k or n * sum(w.shape[0] for w in weights) > k << 22 or k % 8 or not 2 <= len(weights) <= 3:
         return False
     if not (x.is_cuda and x.dtype in (torch.bfloat16, torch.float16) and not torch.is_grad_enabled()
-            and _GUARD.runtime_ok and _native.available()):
+            and _GUARD.runtime_ok and _native.available() and not _native.in_transform()):
         return False
     if not all(w.dtype == x.dtype and w.device == x.device and w.dim() == 2 and w.shape[1] == k and w.stride(1) == 1
                and w.stride(0) % 8 == 0 and w.stride(0) < _GROUP_MAX_STRIDE and w.data_ptr() % 16 == 0

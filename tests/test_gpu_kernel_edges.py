@@ -307,6 +307,29 @@ def test_gemm_group_equals_the_separate_products(M, ns, K, dtype):
                 assert ((got.double() - want.double()).abs() <= 2.0 ** -10 * want.double().abs() + 2.0 ** -24).all()
 
 
+# Under vmap the projections have no memory to launch on: the modules are called, as for any other shape.
+def test_grouped_rows_under_vmap(monkeypatch):
+    from qwen_triton.kernels import matmul, swiglu
+    from qwen_triton.modules import QwenMLP
+
+    monkeypatch.delenv("QWEN_TRITON_STRICT", raising=False)
+    dt = torch.bfloat16
+    torch.manual_seed(0)
+    mlp = QwenMLP(256, 2048).to("cuda", dt).eval()
+    x = _rand(2, 300, 256, dtype=dt, seed=1)
+    with torch.no_grad():
+        assert matmul.linear_group_rows_ok(x[0], [mlp.gate_proj.weight, mlp.up_proj.weight], gated=True)
+        want = torch.stack([mlp(t) for t in x]).double()
+        try:
+            with pytest.warns(RuntimeWarning):
+                got = torch.vmap(mlp)(x).double()
+        finally:
+            matmul._GUARD.reset()
+            swiglu._GUARD.reset()
+    # three bf16 roundings of sums in another order
+    assert (got - want).norm() <= 4 * EPS[dt] * want.norm()
+
+
 # Rows that a product has to copy first are not copied to look at them.
 @pytest.mark.parametrize("form", ["every_other", "overlapping", "expanded", "plain"])
 def test_grouped_rows_are_not_copied_to_look_at_them(form):
