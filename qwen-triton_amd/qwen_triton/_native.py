@@ -160,17 +160,33 @@ def ptr(t: torch.Tensor | None) -> int | None:
 
 _functorch_level, _dispatch_modes = torch._C._functorch.peek_interpreter_stack, torch._C._len_torch_dispatch_stack
 _FAKE_MODE = torch._C._TorchDispatchModeKey.FAKE
+_FUNCTIONALIZE = torch._C._functorch.TransformType.Functionalize
+
+
+def _fake_mode() -> bool:
+    return _dispatch_modes() > 0 and torch._C._get_dispatch_mode(_FAKE_MODE) is not None
 
 
 def in_transform() -> bool:
     """True inside a functorch transform (vmap, jvp, functionalize, ...) or a FakeTensorMode: tensors
-    there stand for others and have no memory to hand to a kernel (``data_ptr()`` raises or is 0)."""
-    return _functorch_level() is not None or (
-        _dispatch_modes() > 0 and torch._C._get_dispatch_mode(_FAKE_MODE) is not None)
+    there may stand for others and have no memory to hand to a kernel (``data_ptr()`` raises or is 0)."""
+    return _functorch_level() is not None or _fake_mode()
+
+
+def _null_pointers() -> bool:
+    """True where such tensors have ``data_ptr()`` 0 (in the other transforms it raises)."""
+    if _functorch_level() is not None and any(
+            level.key() == _FUNCTIONALIZE for level in torch._C._functorch.get_interpreter_stack()):
+        return True
+    return _fake_mode()
 
 
 def stream(device: torch.device | None = None) -> int:
-    """Raw handle of torch's current stream on ``device`` (the stream every kernel is enqueued on)."""
+    """Raw handle of torch's current stream on ``device`` (the stream every kernel is enqueued on).
+
+    Asked for with every launch, so this is where one on tensors without memory is refused."""
+    if _null_pointers():
+        raise Unsupported("inside functionalize or a FakeTensorMode tensors have no memory to launch on")
     if device is None:
         index = torch.cuda.current_device()
     else:

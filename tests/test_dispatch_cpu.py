@@ -334,3 +334,32 @@ def test_structured_mask_matches_the_additive_mask_and_keeps_the_step_start():
     # the dense form: query 0 (position 5) sees keys 2..5 by the window, minus the padding of row 0
     visible = expect[0, 0, 0] == 0
     assert visible.tolist() == [False, False, True, False, False, True, False, False]
+
+
+def test_tensors_without_memory_reach_no_kernel(monkeypatch):
+    """A tensor of a FakeTensorMode, or one inside ``functionalize``, has data_ptr() 0: a launch on it would
+    read address 0. The stream of a launch is refused there, and the operator runs on torch."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+
+    from qwen_triton.kernels import matmul
+
+    monkeypatch.delenv("QWEN_TRITON_STRICT", raising=False)
+    monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda i: 0, raising=False)
+    launched = []
+    monkeypatch.setattr(_native, "call", lambda name, *a: launched.append(name))
+    matmul._GUARD.reset()
+    with FakeTensorMode():
+        x, w = (torch.empty(s, device="cuda", dtype=torch.bfloat16) for s in ((300, 64), (96, 64)))
+        with pytest.warns(RuntimeWarning, match="no memory"), torch.no_grad():
+            out = matmul.triton_matmul(x, w)
+        assert out.shape == (300, 96) and out.dtype == torch.bfloat16
+        assert not matmul.linear_group_rows_ok(x, [w, w])
+    assert matmul._GUARD.runtime_ok and not launched
+    matmul._GUARD.reset()
+    with pytest.raises(_native.Unsupported, match="no memory"):
+        torch.func.functionalize(lambda t: (_native.stream(torch.device("cuda:0")), t)[1])(torch.zeros(2))
+    with pytest.raises(_native.Unsupported, match="no memory"):
+        torch.func.functionalize(torch.vmap(lambda t: (_native.stream(torch.device("cuda:0")), t)[1]))(torch.zeros(2))
+    # elsewhere, and on other tensors inside vmap, a launch is what it was
+    assert _native.stream(torch.device("cuda:0")) == 0
+    torch.vmap(lambda t: (_native.stream(torch.device("cuda:0")), t)[1])(torch.zeros(2))
