@@ -13,7 +13,9 @@ def plain_linears(*modules: nn.Module) -> bool:
     """True when calling each module does nothing but its product: no subclass, replaced ``forward``
     or forward hook that a launch from the weights alone would leave out."""
     hooks = nn.modules.module
-    return not (hooks._global_forward_hooks or hooks._global_forward_pre_hooks) and all(
+    if hooks._global_forward_hooks or hooks._global_forward_pre_hooks or TritonLinear.forward is not _FORWARD:
+        return False
+    return all(
         type(m) is TritonLinear and "forward" not in m.__dict__ and not m._forward_hooks and not m._forward_pre_hooks
         for m in modules)
 
@@ -42,3 +44,6 @@ class TritonLinear(nn.Module):
 
     def extra_repr(self) -> str:
         return f"in_features={self.in_features}, out_features={self.out_features}, bias={self.bias is not None}"
+
+
+_FORWARD = TritonLinear.forward

@@ -363,3 +363,15 @@ def test_tensors_without_memory_reach_no_kernel(monkeypatch):
     # elsewhere, and on other tensors inside vmap, a launch is what it was
     assert _native.stream(torch.device("cuda:0")) == 0
     torch.vmap(lambda t: (_native.stream(torch.device("cuda:0")), t)[1])(torch.zeros(2))
+
+
+def test_plain_linears_sees_a_forward_replaced_on_the_class(monkeypatch):
+    """As on the module itself, in a subclass or through a hook: the module has to be called then."""
+    from qwen_triton.modules.linear import TritonLinear, plain_linears
+
+    lin = TritonLinear(8, 8)
+    assert plain_linears(lin, TritonLinear(8, 4))
+    with monkeypatch.context() as m:
+        m.setattr(TritonLinear, "forward", lambda self, x: -x)
+        assert not plain_linears(lin)
+    assert plain_linears(lin)
