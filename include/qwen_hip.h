@@ -181,6 +181,7 @@ int qh_index_add(void* target, int64_t stride_t, const void* src, int64_t stride
  * rows[r] (token), wsorted[r] (routing weight, dtype), inv[token*top_k + slot]
  * = r; and seg_off[e] (first row of expert e, e = 0..n_experts) and
  * tile_off[e] (first M-tile of expert e for tiles of tile_m rows, prefix sum).
+ * (The workspace is not touched up to 2048 pairs on up to 256 experts.)
  * Replaces the expert_mask / nonzero / where bookkeeping of
  * qwen_triton/modules/moe.py:45-51 (triton_one_hot, qwen_triton/kernels/moe_routing.py:175-200). */
 int64_t qh_moe_dispatch_workspace(int64_t n_tokens, int64_t top_k, int64_t n_experts);
@@ -267,7 +268,9 @@ int qh_moe_scale_bwd(const void* dout, int64_t ldo, const void* D, int64_t ldd, 
  *   B(n,k) = trans_b ? B[k*ldb + n] : B[n*ldb + k]
  * so forward x W^T (0,0), dX = dY W (0,1) and dW = dY^T X (1,1) need no copies.
  * bf16/f16 run on MFMA (32x32x16 tiles; 16x16x32 with a 16-way K split in one
- * workgroup for M <= 128) with fp32 accumulation; f32 runs on VALU.
+ * workgroup for M <= 128) with fp32 accumulation, f32 on the fp32 matrix cores; operands whose rows are not
+ * 16-byte aligned, or lie 2^27 elements apart or more (2^25 for a k-contiguous operand of an output of
+ * several hundred 128x128 tiles), on the VALU.
  * bias has the input dtype; C has out_dtype.
  * Replaces qwen_triton/kernels/matmul.py:64-97 (_matmul_kernel), :100-111 (_bias_add_kernel),
  * :130-200 (forward/backward launchers incl. the per-call transposes at :140, :184). */
@@ -360,7 +363,9 @@ int qh_colsum(const void* X, int64_t ldx, int64_t M, int64_t N, void* out, int d
  * v [B,S,H,Vd] (svb, svs, svh), out (sob, sos, soh), all with unit last
  * stride; g and beta fp32 [B,S,H] with strides (sgb, sgs, sgh); state_out
  * (may be NULL) receives the final fp32 state [B,H,K,Vd] (contiguous, as
- * state_in). K <= 128. One launch for the whole sequence.
+ * state_in). K <= 128. One launch for the whole sequence. bf16 sequences of 320 tokens or more are
+ * solved in chunks of 64: a sequence split into calls then gives the bits of one call only where all of
+ * them are that long and split at multiples of 64 (else it agrees to fp32 rounding of the state).
  * Replaces qwen_triton/kernels/linear_attention.py:54-101
  * (_gated_delta_rule_step_kernel, one launch per token) and the token loop of
  * :130-189 (gated_delta_rule_sequence). */
@@ -492,7 +497,8 @@ int64_t qh_flash_decode_workspace(int64_t B, int64_t Hq, int64_t Hkv, int64_t Sk
  * seqlens (device int32[B], may be NULL) gives each sequence's valid key count
  * (clamped to Sk); with it the launch does not depend on the current length, so
  * a captured decode step can be replayed as the cache grows. Sk then only
- * bounds the keys read and plans the split count.
+ * bounds the keys read and plans the split count. A sequence's result does not
+ * depend on its place in the batch.
  * Replaces the q_len == 1 use of qwen_triton/kernels/flash_attention.py:54-152 made by
  * qwen_triton/modules/attention.py:100-109. */
 int qh_flash_decode(const void* q, int64_t sqb, int64_t sqh, const void* k, int64_t skb, int64_t skh,

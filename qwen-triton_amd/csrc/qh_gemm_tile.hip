@@ -1200,7 +1200,8 @@ __global__ __launch_bounds__(256) void splitk_reduce(const float* __restrict__ P
 // the rounds it needs within 10% of the best fill up to 64 splits (a 128-tile product with
 // K = 151936, the LM head's input gradient for 8192 rows, ran on half the CUs unsplit: 3.26 ms).
 // Below K = 8192 (16384 for fewer than 256 rows, which leave most of a 256-row tile empty) one
-// smaller tile per CU without the partial sums' round trip is faster (us, split / not): weight
+// smaller tile per CU without the partial sums' round trip is faster, or (K from 7000 on, outputs of 1 to 3
+// million) within 8%: 384x3072x8000 44.6 / 47.6, 1024x1024x8000 41 / 33. us, split / not: weight
 // gradients of 5000 rows 1024x1024 41 / 25, 3072x1024 56 / 49, of 11000 rows 45 / 50 and 90 / 97;
 // 2000x1024x8192 59 / 55, 2000x1024x12288 73 / 81; 100 x 1024 x 151936 (the LM head's input gradient
 // of a short text) 3764 on 128x128 tiles, 708 on 64x64.

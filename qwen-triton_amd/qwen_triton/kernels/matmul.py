@@ -234,7 +234,8 @@ def linear_group(x: torch.Tensor, weights: list[torch.Tensor], biases: list[torc
     more rows where ``linear_group_rows_ok`` holds, without norm and residual).
 
     Returns the list of outputs, or ``silu(x @ W_0.T) * (x @ W_1.T)`` when ``gated``; each
-    product is computed and rounded exactly as ``triton_matmul`` would.
+    product is computed and rounded exactly as ``triton_matmul`` would (past 128 rows the gated fp16
+    result may differ from ``silu_mul`` of the two products by one unit in the last place).
 
     ``norm = (weight, eps, one_plus)``: ``x`` holds RMSNorm inputs and the products use
     ``rmsnorm(x)``: the norm weight is folded into the weights once (``round(W * (weight +

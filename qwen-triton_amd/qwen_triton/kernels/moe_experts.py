@@ -11,8 +11,9 @@ all experts, and ``qh_moe_combine`` sums each token's expert rows in ascending
 expert order with the reference's bf16 rounding after every add. No host
 synchronisation; deterministic. With many routed rows per expert the forward
 runs on the 256x256 tile kernels (the training forward below, without keeping
-G and U); sparser routings use ``qh_moe_gemm`` (128-row tiles, gate/up with the
-token gather and SiLU-mul fused, down with the routing-weight scaling fused).
+G and U); sparser routings use ``qh_moe_gemm`` (weights streamed against an expert's
+rows up to 64 of them, else 128-row tiles; gate/up with the token gather and SiLU-mul
+fused, down with the routing-weight scaling fused).
 Both round at the same points.
 
 Training (autograd on) runs ``GroupedExperts``: the same dispatch (with 256-row
