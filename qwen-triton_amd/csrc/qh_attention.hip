@@ -1499,10 +1499,9 @@ __global__ __launch_bounds__(64 * NW) void fa_decode_wg_kernel(const T* __restri
   // parts apart: 2064 positions 542 / 483, 2320 585 / 499, 1016 331 / 306, 1032 343 / 317; at other
   // distances equal (2056: 449 / 450, 4112: 765 / 769). 8 or 16 parts or pseudo-random starts cost 5-10 us a
   // layer at some power-of-two distances; a start by kv-head alone is 506 at 2064.
-  // The softmax sums of part j stay in columns j G .. j G + G - 1 of the MFMA tiles, which hold the query
-  // rows once per part (16 columns, of which one part uses G): a tile's keys are hidden from the columns
-  // of the other parts, so the parts' sums do not depend on the order in which they are walked (0.4 us a
-  // layer, for the parts' combine).
+  // The query rows stand in the MFMA tiles' columns once per part (16 columns, of which one set uses G), and
+  // a part's sums are kept in the lanes of its own columns: so they start afresh with every part, and do not
+  // depend on the order in which the parts are walked (0.5 us a layer, mostly the parts' combine).
   const bool turn = sk_b > kDecodeTurnKeys;
   int part0[NPART + 1];  // first tile of each part; short streams: one part
 #pragma unroll
@@ -1652,10 +1651,31 @@ __global__ __launch_bounds__(64 * NW) void fa_decode_wg_kernel(const T* __restri
     if (ntiles > 0) issue(0, ka);
   }
 
-  float m = -INFINITY, l = 0.f;
-  f32x4 o[DT];
+  float m = -INFINITY, l = 0.f, km = -INFINITY, kl = 0.f;  // of the part being walked, of the kept one
+  f32x4 o[DT], ko[DT];
 #pragma unroll
-  for (int dt = 0; dt < DT; ++dt) o[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int dt = 0; dt < DT; ++dt) o[dt] = ko[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  int part = 0;
+  auto keep = [&]() {  // the sums of `part` into its columns; the next part's start
+    const bool mine = li / G == part;
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) ko[dt][r] = mine ? o[dt][r] : ko[dt][r];
+      o[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    km = mine ? m : km, kl = mine ? l : kl;
+    m = -INFINITY, l = 0.f;
+  };
+  auto enter = [&](int t) {  // tile t comes next
+    int p = 0;
+#pragma unroll
+    for (int j = 1; j < NPART; ++j) p += tile_at(t) >= part0[j];
+    if (p != part) {
+      keep();
+      part = p;
+    }
+  };
 
   auto compute = [&](int t, const v8 (&kf)[2][KD]) {
     const T* Vt = Vs[w][t % NS];
@@ -1665,16 +1685,12 @@ __global__ __launch_bounds__(64 * NW) void fa_decode_wg_kernel(const T* __restri
       s0 = mma16<T>(kf[0][kd], qf[kd], s0);
       s1 = mma16<T>(kf[1][kd], qf[kd], s1);
     }
-    const int tt = tile_at(t), kbase = (w + tt * NW) * BN + 4 * lg;
-    int part = 0;
-#pragma unroll
-    for (int j = 1; j < NPART; ++j) part += tt >= part0[j];
-    const int kend = li / G == part ? sk_b : 0;  // keys that this column sees
+    const int kbase = tile_row(t) + 4 * lg;
     float x[8];
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      x[r] = kbase + r < kend ? s0[r] * scale_log2 : -INFINITY;
-      x[4 + r] = kbase + 16 + r < kend ? s1[r] * scale_log2 : -INFINITY;
+      x[r] = kbase + r < sk_b ? s0[r] * scale_log2 : -INFINITY;
+      x[4 + r] = kbase + 16 + r < sk_b ? s1[r] * scale_log2 : -INFINITY;
     }
     float mx = fmaxf(fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3])), fmaxf(fmaxf(x[4], x[5]), fmaxf(x[6], x[7])));
     mx = fmaxf(mx, __shfl_xor(mx, 16));
@@ -1740,6 +1756,7 @@ __global__ __launch_bounds__(64 * NW) void fa_decode_wg_kernel(const T* __restri
       __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
     }
     patch(t, ka);
+    enter(t);
     compute(t, ka);
     if (t + 1 < ntiles) {
       if (t + 2 < ntiles) {
@@ -1749,18 +1766,20 @@ __global__ __launch_bounds__(64 * NW) void fa_decode_wg_kernel(const T* __restri
         __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
       }
       patch(t + 1, kb);
+      enter(t + 1);
       compute(t + 1, kb);
     }
   }
-  l += __shfl_xor(l, 16);
-  l += __shfl_xor(l, 32);
+  keep();
+  kl += __shfl_xor(kl, 16);
+  kl += __shfl_xor(kl, 32);
   if (li < NP) {
     float* co = reinterpret_cast<float*>(&Vs[w][0][0]) + li * COLD + 4 * lg;  // (the wave has read its V stages)
 #pragma unroll
-    for (int dt = 0; dt < DT; ++dt) *reinterpret_cast<f32x4*>(co + dt * 16) = o[dt];
+    for (int dt = 0; dt < DT; ++dt) *reinterpret_cast<f32x4*>(co + dt * 16) = ko[dt];
     if (lg == 0) {
-      cml[w][li][0] = m;
-      cml[w][li][1] = l;
+      cml[w][li][0] = km;
+      cml[w][li][1] = kl;
     }
   }
   __syncthreads();

@@ -667,6 +667,22 @@ def test_decode_attention_does_not_depend_on_the_slot(Hq, Hkv, Sk):
     assert ((out[:n].cpu().double() - ref).abs() <= bound).all()
 
 
+@pytest.mark.parametrize("Hq,Hkv", [(16, 8), (64, 8)])
+@pytest.mark.parametrize("key", [5, 900, 1400, 2000])
+def test_decode_attention_of_an_infinite_value(Hq, Hkv, key):
+    """An infinity among the values reaches its own output dimension as an infinity, whatever part of the
+    stream it lies in, and nothing else."""
+    from qwen_triton.kernels.flash_attention import flash_decode
+
+    B, Sk, D, dt = 66, 2050, 128, torch.bfloat16
+    q, k, v = (_rand(B, h, s, D, dtype=dt, seed=i) for i, (h, s) in enumerate([(Hq, 1), (Hkv, Sk), (Hkv, Sk)]))
+    v[:, 3, key, 17] = float("inf")
+    out = flash_decode(q, k, v, D ** -0.5, Hq // Hkv).view(B, Hkv, Hq // Hkv, D)
+    assert (out[:, 3, :, 17] == float("inf")).all()
+    out[:, 3, :, 17] = 0
+    assert torch.isfinite(out).all()
+
+
 # The step that prepares its own rows: the same, for 8 wavefronts (32 sequences) and 4.
 @pytest.mark.parametrize("B,Sk,pos", [(32, 1100, 1099), (32, 520, 100), (72, 2050, 1300)])
 def test_decode_step_does_not_depend_on_the_slot(B, Sk, pos):
