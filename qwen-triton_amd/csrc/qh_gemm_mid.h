@@ -120,8 +120,8 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void gemm_mid_kernel(const T* __
     if (K - WK * t * BK < WK * BK) {  // (uniform) the round with the last k-tile: K may end inside one
       const int vk = K - (ks + WK * t) * BK;
       if (vk > 0 && vk < BK) {
-        TA::zero_k_tail(S, vk);
-        TB::zero_k_tail(S + TA::ELEMS, vk);
+        TA::zero_k_tail(S, vk, threadIdx.x % (64 * NW));
+        TB::zero_k_tail(S + TA::ELEMS, vk, threadIdx.x % (64 * NW));
       }
       __syncthreads();
       if (vk <= 0) break;  // no k-tile for this slice in the last round

@@ -244,8 +244,8 @@ __global__ __launch_bounds__(NTHR) void gemm_tile_kernel(P p) {
     const int vk = c.K - kt * BK;
     if (vk < BK) {
       T* S = stage(kt);
-      TA::zero_k_tail(S, vk);
-      TB::zero_k_tail(S + TA::ELEMS, vk);
+      TA::zero_k_tail(S, vk, threadIdx.x);
+      TB::zero_k_tail(S + TA::ELEMS, vk, threadIdx.x);
       __syncthreads();
     }
   };

@@ -115,9 +115,9 @@ struct NTile {
 #pragma unroll
     for (int i = 0; i < PW; ++i) lds_dma16(rowp[i] + k0 + kc, lds + (uint32_t)(wid + NW * i) * 1024u);
   }
-  // Zero the k chunks at or past vk (all rows).
-  static __device__ __forceinline__ void zero_k_tail(T* S, int vk) {
-    for (int idx = threadIdx.x % (64 * NW); idx < ROWS * CPR; idx += 64 * NW) {
+  // Zero the k chunks at or past vk (all rows); tid: the thread among the tile's 64 NW.
+  static __device__ __forceinline__ void zero_k_tail(T* S, int vk, int tid) {
+    for (int idx = tid; idx < ROWS * CPR; idx += 64 * NW) {
       const int r = idx / CPR, c = idx % CPR;
       if (E * c >= vk) *reinterpret_cast<uint4*>(S + r * BK + E * (c ^ sw(r))) = make_uint4(0, 0, 0, 0);
     }
@@ -207,8 +207,8 @@ struct TTile {
       issue(lds, at, k0, vcols, vk, vo2, wid + NW / 2);
     }
   }
-  static __device__ __forceinline__ void zero_k_tail(T* S, int vk) {
-    for (int idx = threadIdx.x % (64 * NW); idx < BK * CPR; idx += 64 * NW) {
+  static __device__ __forceinline__ void zero_k_tail(T* S, int vk, int tid) {
+    for (int idx = tid; idx < BK * CPR; idx += 64 * NW) {
       const int kr = idx / CPR;
       if (kr >= vk) *reinterpret_cast<uint4*>(S + idx * 8) = make_uint4(0, 0, 0, 0);
     }
@@ -267,8 +267,8 @@ struct TTileF32 {
       lds_dma16(at(col, k0 + kr), lds + (uint32_t)n * 1024u);
     }
   }
-  static __device__ __forceinline__ void zero_k_tail(float* S, int vk) {
-    for (int idx = threadIdx.x % (64 * NW); idx < BK * CPR; idx += 64 * NW)
+  static __device__ __forceinline__ void zero_k_tail(float* S, int vk, int tid) {
+    for (int idx = tid; idx < BK * CPR; idx += 64 * NW)
       if (krow(idx / CPR) >= vk) *reinterpret_cast<uint4*>(S + idx * 4) = make_uint4(0, 0, 0, 0);
   }
   static __device__ __forceinline__ f32x4 frag(const float* S, int r0, int g) {
