@@ -1425,9 +1425,11 @@ __global__ __launch_bounds__(256) void fa_decode_combine(const float* __restrict
 // tile's end (key p, and the rows past the last key that the tile load clamps
 // to it) are rewritten in the V stage. So no load waits for the stores, whose
 // bytes are those the patch supplies.
-// Keys up to which a stream is walked in order: nothing was gained by parting shorter ones (64 sequences of
-// 300 or 500 keys, four layers: 184 and 222 us either way).
-constexpr int kDecodeTurnKeys = 512;
+// Keys up to which a stream is walked in order. Four layers of 64 sequences, in order / in parts, us: caches of
+// 536, 680, 800, 920 and 992 positions 212 / 216, 236 / 240, 254 / 259, 275 / 278, 282 / 286; 1016 325 / 304, 1032
+// 339 / 317. A launch of streams up to here has a kernel without the parts' code (TURN false), whose registers
+// and combine cost steps of 33 to 500 keys 1 to 2%.
+constexpr int kDecodeTurnKeys = 960;
 
 template <typename T, bool PREP>
 using kv_ptr = typename std::conditional<PREP, const T*, const T* __restrict__>::type;
@@ -1454,7 +1456,9 @@ struct DecodePrepArgs {
 // last-level cache); short caches, read again at the next step, keep the default policy.
 // NW wavefronts per workgroup (8 for short caches of more than 4 tiles, so that no
 // wave computes two tiles one after the other).
-template <typename T, int DP, int G, bool PREP = false, typename C = float, bool NTKV = true, int NW = 4>
+// TURN: streams may be longer than kDecodeTurnKeys (the parts below).
+template <typename T, int DP, int G, bool PREP = false, typename C = float, bool NTKV = true, int NW = 4,
+          bool TURN = true>
 __global__ __launch_bounds__(64 * NW) void fa_decode_wg_kernel(const T* __restrict__ Q, int64_t sqb, int64_t sqh,
                                                           kv_ptr<T, PREP> K, int64_t skb, int64_t skh,
                                                           int64_t sks, kv_ptr<T, PREP> V, int64_t svb,
@@ -1464,7 +1468,7 @@ __global__ __launch_bounds__(64 * NW) void fa_decode_wg_kernel(const T* __restri
                                                           const DecodePrepArgs<T, C> pa) {
   static_assert(G >= 1 && G <= 8, "query heads per kv-head");
   constexpr int BN = 32, NS = 2;
-  constexpr int NPART = G <= 4 ? 4 : 2;  // parts of a long stream, G of the 16 MFMA columns each
+  constexpr int NPART = !TURN ? 1 : G <= 4 ? 4 : 2;  // parts of a long stream, G of the 16 MFMA columns each
   constexpr int NP = NPART * G;
   constexpr int CPR = DP / 8;    // 16-byte chunks per row
   constexpr int RPI = 64 / CPR;  // rows per 1 KiB load instruction
@@ -1502,7 +1506,7 @@ __global__ __launch_bounds__(64 * NW) void fa_decode_wg_kernel(const T* __restri
   // The query rows stand in the MFMA tiles' columns once per part (16 columns, of which one set uses G), and
   // a part's sums are kept in the lanes of its own columns: so they start afresh with every part, and do not
   // depend on the order in which the parts are walked (0.5 us a layer, mostly the parts' combine).
-  const bool turn = sk_b > kDecodeTurnKeys;
+  const bool turn = TURN && sk_b > kDecodeTurnKeys;
   int part0[NPART + 1];  // first tile of each part; short streams: one part
 #pragma unroll
   for (int j = 0; j <= NPART; ++j) part0[j] = j == 0 ? 0 : (turn ? j * ntiles / NPART : ntiles);
@@ -2142,14 +2146,20 @@ extern "C" int qh_flash_decode(const void* q, int64_t sqb, int64_t sqh, const vo
   const float sl2 = scale * kLog2e;
   if (decode_on_chip(B, Hkv, dp)) {
     // many sequences: one workgroup per (b, kv-head), combined in LDS
-#define QH_WG(T, GV)                                                                                              \
-  fa_decode_wg_kernel<T, 128, GV><<<(unsigned)(B * Hkv), 256, 0, st>>>(                                         \
+#define QH_WG_T(T, GV, TURN)                                                                                      \
+  fa_decode_wg_kernel<T, 128, GV, false, float, true, 4, TURN><<<(unsigned)(B * Hkv), 256, 0, st>>>(              \
       (const T*)q, sqb, sqh, (const T*)k, skb, skh, sks, (const T*)v, svb, svh, svs, (T*)o, lse, seqlens, (int)Hkv, \
       (int)Sk, (int)D, sl2, DecodePrepArgs<T, float>{})
+#define QH_WG(T, GV)                                      \
+  {                                                       \
+    if (Sk > kDecodeTurnKeys) QH_WG_T(T, GV, true);       \
+    else QH_WG_T(T, GV, false);                           \
+  }
 #define QH_WG_G(T) \
-  if (groups == 1) QH_WG(T, 1); else if (groups == 2) QH_WG(T, 2); else if (groups == 4) QH_WG(T, 4); else QH_WG(T, 8);
+  if (groups == 1) QH_WG(T, 1) else if (groups == 2) QH_WG(T, 2) else if (groups == 4) QH_WG(T, 4) else QH_WG(T, 8)
     if (dtype == QH_BF16) { QH_WG_G(bf16_t) } else { QH_WG_G(f16_t) }
 #undef QH_WG_G
+#undef QH_WG_T
 #undef QH_WG
     QH_CHECK_LAUNCH("qh_flash_decode");
     return QH_OK;
@@ -2308,27 +2318,29 @@ extern "C" int qh_flash_decode_prepare(const void* q, int64_t sq, const void* k,
   hipStream_t st = (hipStream_t)stream;
   const float sl2 = scale * kLog2e;
   const int groups = (int)(Hq / Hkv);
+#define QH_WGP_K(T, C, GV, NTKV, NW, TURN)                                                                          \
+  fa_decode_wg_kernel<T, 128, GV, true, C, NTKV, NW, TURN><<<(unsigned)(B * Hkv), 64 * NW, 0, st>>>(               \
+      (const T*)o, 0, 0, (const T*)k_cache, kcb, kch, kcs, (const T*)v_cache, vcb, vch, vcs, (T*)o, lse, seqlens,  \
+      (int)Hkv, (int)Sk, (int)D, sl2, pa)
 #define QH_WGP(T, C, GV)                                                                                           \
   {                                                                                                                \
     DecodePrepArgs<T, C> pa{(const T*)q, (const T*)k, (const T*)v, sq, sk, sv, qw, kw, wdtype, eps,               \
                             one_plus ? 1.f : 0.f, (const C*)cos, (const C*)sin, scb, (int)cos_batch, (int)half,    \
                             (int)rot, positions, cap};                                                            \
-    if (B * Hkv >= kDecodeWgMinSeqs)                                                                              \
-      fa_decode_wg_kernel<T, 128, GV, true, C><<<(unsigned)(B * Hkv), 256, 0, st>>>(                             \
-          (const T*)o, 0, 0, (const T*)k_cache, kcb, kch, kcs, (const T*)v_cache, vcb, vch, vcs, (T*)o, lse,      \
-          seqlens, (int)Hkv, (int)Sk, (int)D, sl2, pa);                                                           \
-    else if (GV <= 4 && Sk > kDecodeWgShortKeys && B * Hkv >= kDecodeWgMidNt)                                      \
-      fa_decode_wg_kernel<T, 128, GV, true, C, true, (GV <= 4 ? 8 : 4)><<<(unsigned)(B * Hkv), 64 * (GV <= 4 ? 8 : 4), 0, st>>>( \
-          (const T*)o, 0, 0, (const T*)k_cache, kcb, kch, kcs, (const T*)v_cache, vcb, vch, vcs, (T*)o, lse,      \
-          seqlens, (int)Hkv, (int)Sk, (int)D, sl2, pa);                                                           \
-    else if (GV <= 4 && Sk > 4 * 32)                                                                               \
-      fa_decode_wg_kernel<T, 128, GV, true, C, false, (GV <= 4 ? 8 : 4)><<<(unsigned)(B * Hkv), 64 * (GV <= 4 ? 8 : 4), 0, st>>>( \
-          (const T*)o, 0, 0, (const T*)k_cache, kcb, kch, kcs, (const T*)v_cache, vcb, vch, vcs, (T*)o, lse,      \
-          seqlens, (int)Hkv, (int)Sk, (int)D, sl2, pa);                                                           \
-    else                                                                                                           \
-      fa_decode_wg_kernel<T, 128, GV, true, C, false><<<(unsigned)(B * Hkv), 256, 0, st>>>(                      \
-          (const T*)o, 0, 0, (const T*)k_cache, kcb, kch, kcs, (const T*)v_cache, vcb, vch, vcs, (T*)o, lse,      \
-          seqlens, (int)Hkv, (int)Sk, (int)D, sl2, pa);                                                           \
+    constexpr int NW8 = GV <= 4 ? 8 : 4;                                                                          \
+    const bool turn = Sk > kDecodeTurnKeys;                                                                       \
+    if (B * Hkv >= kDecodeWgMinSeqs) {                                                                            \
+      if (turn) QH_WGP_K(T, C, GV, true, 4, true);                                                                \
+      else QH_WGP_K(T, C, GV, true, 4, false);                                                                    \
+    } else if (GV <= 4 && Sk > kDecodeWgShortKeys && B * Hkv >= kDecodeWgMidNt) {                                 \
+      if (turn) QH_WGP_K(T, C, GV, true, NW8, true);                                                              \
+      else QH_WGP_K(T, C, GV, true, NW8, false);                                                                  \
+    } else if (GV <= 4 && Sk > 4 * 32) {                                                                          \
+      if (turn) QH_WGP_K(T, C, GV, false, NW8, true);                                                             \
+      else QH_WGP_K(T, C, GV, false, NW8, false);                                                                 \
+    } else {                                                                                                      \
+      QH_WGP_K(T, C, GV, false, 4, false);                                                                        \
+    }                                                                                                             \
   }
 #define QH_WGP_G(T, C) \
   if (groups == 1) QH_WGP(T, C, 1) else if (groups == 2) QH_WGP(T, C, 2) else if (groups == 4) QH_WGP(T, C, 4) else QH_WGP(T, C, 8)
@@ -2339,6 +2351,7 @@ extern "C" int qh_flash_decode_prepare(const void* q, int64_t sq, const void* k,
   }
 #undef QH_WGP_G
 #undef QH_WGP
+#undef QH_WGP_K
   QH_CHECK_LAUNCH("qh_flash_decode_prepare");
   return QH_OK;
 }

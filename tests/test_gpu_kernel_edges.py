@@ -643,15 +643,15 @@ def test_moe_tokens_on_few_experts_are_not_streamed_twice():
 
 # One workgroup per (sequence, kv-head) starts long streams at different parts: a sequence's result may not
 # depend on its place in the batch (equal sequences in slots of every starting part), and it is right where
-# parts hold no tile, one or many; lengths on both sides of the 512 keys up to which a stream is not parted.
+# parts hold no tile, one or many; lengths on both sides of the 960 keys up to which a stream is not parted.
 @pytest.mark.parametrize("Hq,Hkv", [(8, 8), (16, 8), (32, 8), (64, 8)])
-@pytest.mark.parametrize("Sk", [513, 640, 1111, 2050])
+@pytest.mark.parametrize("Sk", [700, 961, 1111, 2050])
 def test_decode_attention_does_not_depend_on_the_slot(Hq, Hkv, Sk):
     from qwen_triton.kernels.flash_attention import flash_decode
 
     n, reps, D, dt = 6, 11, 128, torch.bfloat16  # 6 sequences, each in 11 slots
     q, k, v = (_rand(n, h, s, D, dtype=dt, seed=i) for i, (h, s) in enumerate([(Hq, 1), (Hkv, Sk), (Hkv, Sk)]))
-    lens = torch.tensor([Sk, 512, 513, Sk - 1, 33, (Sk + 513) // 2], dtype=torch.int32).clamp(max=Sk)
+    lens = torch.tensor([Sk, 960, 961, Sk - 1, 33, (Sk + 961) // 2], dtype=torch.int32).clamp(max=Sk)
     slot = torch.arange(n * reps) % n
     i = slot.cuda()
     out = flash_decode(q[i], k[i].contiguous(), v[i].contiguous(), D ** -0.5, Hq // Hkv, seqlens=lens[slot].cuda())
@@ -684,7 +684,7 @@ def test_decode_attention_of_an_infinite_value(Hq, Hkv, key):
 
 
 # The step that prepares its own rows: the same, for 8 wavefronts (32 sequences) and 4.
-@pytest.mark.parametrize("B,Sk,pos", [(32, 1100, 1099), (32, 520, 100), (72, 2050, 1300)])
+@pytest.mark.parametrize("B,Sk,pos", [(32, 1100, 1099), (32, 970, 100), (32, 600, 599), (72, 2050, 1300)])
 def test_decode_step_does_not_depend_on_the_slot(B, Sk, pos):
     from qwen_triton import _native
 
