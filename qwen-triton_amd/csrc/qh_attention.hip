@@ -417,22 +417,22 @@ __global__ __launch_bounds__(256) void fa_fwd_kernel(const T* __restrict__ Q, in
   const TileLoader<T, BN, DP> kload(sks, D), vload(svs, D);
   // stage of tile r + g of the round from r on (KW = 2: rounds of two tiles from it0 on)
   auto stage = [&](int r, int g) { return KW > 1 ? 2 * g + ((r - it0) >> 1 & 1) : r & 1; };
-  auto load = [&](int r) {
+  auto load = [&](int r, int row0, int buf) {  // tiles from r on, at row row0; KW = 1: into stage buf
 #pragma unroll
     for (int g = 0; g < KW; ++g)
       if (r + g < ntiles) {
-        kload.load(Ks[stage(r, g)], Kb, sks, (r + g) * BN, Sk);
-        vload.load(Vs[stage(r, g)], Vb, svs, (r + g) * BN, Sk);
+        kload.load(Ks[KW > 1 ? stage(r, g) : buf], Kb, sks, row0 + g * BN, Sk);
+        vload.load(Vs[KW > 1 ? stage(r, g) : buf], Vb, svs, row0 + g * BN, Sk);
       }
   };
-  load(it0);
+  load(it0, it0 * BN, it0 & 1);
   for (int r = it0; r < ntiles; r += KW) {
     const int it = r + kg;
     const int kv0 = it * BN;
     const int buf = stage(r, kg);
     __builtin_amdgcn_s_waitcnt(0);  // this thread's loads of the round have landed
     __syncthreads();                // ... and everyone else's; the round before is fully consumed
-    load(r + KW);
+    load(r + KW, (r + KW) * BN, buf ^ 1);
     if (KW > 1 && it >= ntiles) break;  // the last round: no tile for this group
     // wave-uniform: does any key of this tile lie past a query's limit?
     // (one code path for both: two inlined copies of the tile would hold the
