@@ -1882,6 +1882,7 @@ extern "C" int qh_lmce_fwd(const void* X, int64_t ldx, const void* W, int64_t ld
   QH_CHECK_ARG(dtype == QH_BF16 || dtype == QH_F16, "qh_lmce_fwd: bf16/f16 only");
   QH_CHECK_ARG(aligned16(X) && aligned16(W) && ldx % 8 == 0 && ldw % 8 == 0 && H % 8 == 0 && ldx >= H && ldw >= H,
                "qh_lmce_fwd: X and W must be 16-byte aligned k-contiguous rows with H, ldx, ldw multiples of 8");
+  QH_CHECK_ARG(ldx < kTileMaxLd && ldw < kTileMaxLd, "qh_lmce_fwd: rows of X or W 2^27 or more elements apart");
   QH_CHECK_ARG(ws_bytes >= qh_lmce_workspace(N, V), "qh_lmce_fwd: workspace %lld < %lld", (long long)ws_bytes,
                (long long)qh_lmce_workspace(N, V));
   if (N == 0) return qh_zero(loss_out, 4, stream) || qh_zero(nvalid_out, 4, stream);
@@ -1999,6 +2000,7 @@ extern "C" int qh_gemm_acc(int trans_a, int trans_b, int64_t M, int64_t N, int64
   QH_CHECK_ARG(aligned16(A) && aligned16(B) && lda % 8 == 0 && ldb % 8 == 0 && (trans_a ? M % 8 == 0 : K % 8 == 0) &&
                    (trans_b ? N % 8 == 0 : K % 8 == 0),
                "qh_gemm_acc: 16-byte aligned operands with contiguous extents and strides multiples of 8 required");
+  QH_CHECK_ARG(lda < kTileMaxLd && ldb < kTileMaxLd, "qh_gemm_acc: operand rows 2^27 or more elements apart");
   if (M == 0 || N == 0 || K == 0) return QH_OK;
   hipStream_t st = (hipStream_t)stream;
   int rc = QH_OK;

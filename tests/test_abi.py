@@ -135,6 +135,17 @@ def test_fused_loss_refuses_rows_past_its_lane_offsets(ldx, ldw):
                      4096, 1 << 30, _native.BF16, 0)
 
 
+@pytest.mark.parametrize("wide", [0, 1])
+def test_loss_products_refuse_rows_past_their_lane_offsets(wide):
+    ld = [64, 64]
+    ld[wide] = 1 << 27
+    with pytest.raises(_native.NativeUnsupported, match="elements apart"):
+        _native.call("qh_lmce_fwd", 4096, ld[0], 4096, ld[1], 4096, 512, 1024, 64, -100, 4096, 4096, 4096, 4096, 4096,
+                     1 << 30, _native.BF16, 0)
+    with pytest.raises(_native.NativeUnsupported, match="elements apart"):
+        _native.call("qh_gemm_acc", 0, 0, 256, 256, 64, 4096, ld[0], 4096, ld[1], 4096, 256, _native.BF16, 0)
+
+
 def test_grouped_products_leave_split_k_alone():
     n = (ctypes.c_int64 * 2)(3072, 3072)
     ok = lambda K: _native.call("qh_gemm_group_ok", 517, K, 2, ctypes.addressof(n), 1)  # noqa: E731
